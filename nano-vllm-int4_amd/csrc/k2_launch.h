@@ -14,4 +14,10 @@ hipError_t k2_prefill_launch(const int8_t* a, const int8_t* w, const void* sa, c
                              bool sw_grouped, void* out, bool out_fp32, bool w_tiled, int M, int N, int K,
                              hipStream_t st);
 
+// Mid-sized grouped W4A4 GEMM (M > 32): 32..48 x 64..128 tiles, weights in
+// registers.  Same arguments and contract.
+hipError_t k2_mid_launch(const int8_t* a, const int8_t* w, const void* sa, const void* sw,
+                         bool sw_grouped, void* out, bool out_fp32, bool w_tiled, int M, int N, int K,
+                         hipStream_t st);
+
 }  // namespace nv4

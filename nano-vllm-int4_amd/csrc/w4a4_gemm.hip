@@ -22,8 +22,8 @@
 // as 1 KiB in lane order), which lets every weight load be whole cache
 // lines; the results are the same bits.
 //
-// Three kernels, no split-K, no atomics:
-//  * k2_dec (M <= 64): one workgroup per 16 output columns (two 16-column
+// Four kernels, no split-K, no atomics:
+//  * k2_dec (M <= 32, and M <= 64 on narrow N): one workgroup per 16 output columns (two 16-column
 //    blocks when one each would put two workgroups, each reading all of the
 //    activations, on some CUs) and all M rows.
 //    Its 8 or 16 waves each take one K group per round, compute the exact
@@ -32,7 +32,8 @@
 //    Loads run several rounds ahead.
 //  * k2_wide (M <= 32, wide N): waves own column blocks over the whole K,
 //    activations widened once per CU into LDS.
-//  * k2_prefill (M > 64, w4a4_prefill.hip): LDS-staged 128x128 tiles.
+//  * k2_mid (M > 32, w4a4_mid.hip): 32..48 x 64..128 tiles, whole K per wave.
+//  * k2_prefill (M >= 2048, w4a4_prefill.hip): LDS-staged 128x128 tiles.
 #include "k2_launch.h"
 #include "norm_ops.h"
 #include "nv4_common.h"
@@ -726,8 +727,18 @@ hipError_t dispatch(const int8_t* a, const int8_t* w, const void* sa, const void
     }
     if (M <= 16) return launch_dec<1, TW, false, SG, OF>(a, w, sa, sw, out, M, N, K, st);
     if (M <= 32) return launch_dec<2, TW, false, SG, OF>(a, w, sa, sw, out, M, N, K, st);
-    if (M <= 48) return launch_dec<3, TW, false, SG, OF>(a, w, sa, sw, out, M, N, K, st);
-    if (M <= 64) return launch_dec<4, TW, false, SG, OF>(a, w, sa, sw, out, M, N, K, st);
+    // Up to five 16 x 16 blocks per CU the K-split waves of k2_dec beat the
+    // mid-sized kernel's whole-K waves (us per call, k2_dec / k2_mid: o at M =
+    // 33 / 64: 6.9 / 9.9 and 8.5 / 9.7; down 14.4 / 22.2 and 19.2 / 22.7; qkv at
+    // 48: 10.0 / 9.9, and beyond the line qkv at 64: 15.3 / 9.9, gate_up at 33:
+    // 22.1 / 16.6).
+    if (M <= 64 && (int64_t)((M + 15) / 16) * ((N + 15) / 16) <= 5LL * device_cu_count())
+        return M <= 48 ? launch_dec<3, TW, false, SG, OF>(a, w, sa, sw, out, M, N, K, st)
+                       : launch_dec<4, TW, false, SG, OF>(a, w, sa, sw, out, M, N, K, st);
+    // From M = 2048 the 128 x 128 tiles fill the chip and move fewer bytes (o /
+    // qkv / down / gate_up at 2048: 59 / 93 / 167 / 317 us against 65 / 95 /
+    // 172 / 326; at 1024 46 / 59 / 125 / 169 against 34 / 49 / 89 / 163).
+    if (M < 2048) return k2_mid_launch(a, w, sa, sw, SG, out, OF, TW, M, N, K, st);
     return k2_prefill_launch(a, w, sa, sw, SG, out, OF, TW, M, N, K, st);
 }
 
