@@ -18,8 +18,8 @@
 // bf16 MFMA as in the fp8 kernel; one VALU fma per output and group remains.
 //
 // Operand format (written by i4_to_f6_tiles into the caller's workspace, or
-// for weights converted once by nv4_w4a4_weights_to_f6): rows in tiles of 128; per tile and group one 12 KiB block laid out as LDS
-// reads it.  A group row's 128 codes are four quarters of 32 (k = 32q ..
+// for weights converted once by nv4_w4a4_weights_to_f6): rows in tiles of
+// 128; per tile and group one 12 KiB block laid out as LDS reads it.  A group row's 128 codes are four quarters of 32 (k = 32q ..
 // 32q + 31, 24 bytes each, code k at bit 6k of the quarter, little endian),
 // and each quarter is split into its first 16 bytes (P) and last 8 (R):
 //   P[q][row] at q * 2048 + row * 16,  R[q][row] at 8192 + q * 1024 + row * 8.
@@ -33,8 +33,17 @@
 // layout as fp8: lane l holds C[8*(i/4) + 4*(l/32) + i%4][l%32], i = 0..15.
 //
 // Workgroup = 4 waves, 128 x 128 output tile, whole K, two workgroups per
-// CU, XCD-aware tile order, a two-stage operand ring with one barrier per
-// group and the bf16 scales in 8-group windows (as the fp8 kernel).
+// CU, XCD-aware tile order, and the bf16 scales in 8-group windows.  Operands
+// go through a three-stage LDS ring, loaded three groups ahead, with one
+// barrier per group; a wave reads an operand of the next group right after
+// its last use in this one, and every MFMA is followed by a third of the
+// previous block's fma chain, so LDS, matrix cores and vector ALUs work at the
+// same time.  Against a two-stage ring with a group's reads, MFMAs and fmas in
+// turn (us per call with the conversion): M = 4096 qkv 113 -> 103, o 78.8 ->
+// 72.9, gate_up 402 -> 390, down 206 -> 196; M = 1024 o 34.3 -> 30.4, down 82 ->
+// 69.  What bounds it now: the chip's power at large M (gate_up at 4096 rows
+// takes 330 us on zero codes and 286 without the operand loads), one
+// workgroup's own 0.42 us per group while tiles are fewer than CUs.
 #include "nv4_common.h"
 
 namespace nv4 {
@@ -45,11 +54,13 @@ constexpr int F6_BLOCK = 12 * 1024;                     // one operand tile, one
 constexpr int F6_R = 8192;                              // R part of a block
 constexpr int F6_STAGE = 2 * F6_BLOCK;                  // A block then W block
 constexpr int F6_WSZ = 8 * (F6_BM + F6_BN) * 2;         // 8 groups x (sa[128], sw[128]) bf16
-static_assert(2 * F6_STAGE + 2 * F6_WSZ == 56 * 1024, "56 KiB of LDS: two workgroups per CU");
+static_assert(3 * F6_STAGE + 2 * F6_WSZ == 80 * 1024, "80 KiB of LDS: two workgroups per CU");
+constexpr int F6_OOR = 0x7fffff00;                      // scalar offset past every resource
 constexpr int F6_GM = 8;                                // M-tiles per column sweep
 constexpr int F6_RSRC_WORD3 = 0x00020000;               // buffer resource word 3 (CDNA): 32-bit data format
 constexpr int F6_FMT = 3;                               // f8f6f4 operand format: e3m2
 
+typedef short v4s __attribute__((ext_vector_type(4)));
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(3))) void* lds_ptr;
 
@@ -135,17 +146,40 @@ __device__ __forceinline__ void f6_tile(int tm, int tn, int& mt, int& nt) {
     nt = r / gm;
 }
 
+// 16 bytes per lane from a buffer straight into LDS (lane l's at lds + 16 l;
+// out-of-range lanes write zeros), as volatile asm: the compiler would order
+// every later LDS read behind the load (it tracks few of them apart), while
+// here stages in flight are never the ones being read.  The caller waits
+// (vmcnt) and passes a barrier before reading.
+__device__ __forceinline__ void f6_load_lds(const v4u& rsrc, uint32_t voff, uint32_t soff, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff),
+                 "s"(rsrc), "s"(soff)
+                 : "memory");
+}
+__device__ __forceinline__ v4u f6_rsrc(const void* p, uint32_t bytes) {
+    const uint64_t x = reinterpret_cast<uint64_t>(p);
+    return v4u{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)x),
+               (uint32_t)__builtin_amdgcn_readfirstlane((int)((x >> 32) & 0xffffu)),
+               (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), (uint32_t)F6_RSRC_WORD3};
+}
+__device__ __forceinline__ uint32_t f6_lds(const void* p) {
+    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
+}
+template <int N>
+__device__ __forceinline__ void f6_barrier() {  // all but the N youngest loads done, then the workgroup's barrier
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
 template <bool SG, bool OF, bool WIN>
 __global__ void __launch_bounds__(F6_T, 2)
 k2_prefill_f6(const uint8_t* __restrict__ a, const uint8_t* __restrict__ w, const uint16_t* __restrict__ sa,
               const uint16_t* __restrict__ sw, void* __restrict__ out, int M, int N, int K, int tm, int tn) {
-    // Two operand stages (A block then W block) and the scales (8-group
-    // windows, or one slot per group), as separate arrays so that reads of
-    // one stage are not ordered behind the direct-to-LDS loads in flight into
-    // the other.
-    __shared__ __align__(16) uint8_t st0[F6_STAGE];
-    __shared__ __align__(16) uint8_t st1[F6_STAGE];
-    __shared__ __align__(16) uint16_t win[WIN ? F6_WSZ : 2 * (F6_BM + F6_BN)];
+    // Three operand stages (A block then W block) and the scales (8-group
+    // windows, or one slot per group).
+    __shared__ __align__(16) uint8_t st[3 * F6_STAGE];
+    __shared__ __align__(16) uint16_t win[WIN ? F6_WSZ : 4 * (F6_BM + F6_BN)];
     int mt, nt;
     f6_tile(tm, tn, mt, nt);
     const int m0 = mt * F6_BM, n0 = nt * F6_BN;
@@ -157,54 +191,44 @@ k2_prefill_f6(const uint8_t* __restrict__ a, const uint8_t* __restrict__ w, cons
     // Direct-to-LDS staging: load i (0..2) of wave w copies the 1 KiB at
     // (3w + i) * 1024 of the group's A block (then of its W block), lane l
     // the 16 bytes at l * 16.  Buffer resources over the tile's G blocks, so
-    // the loads take a fixed lane offset and the group offset as a scalar.
-    const __amdgpu_buffer_rsrc_t rsa = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint8_t*>(a + (int64_t)mt * G * F6_BLOCK), (short)0, G * F6_BLOCK, F6_RSRC_WORD3);
-    const __amdgpu_buffer_rsrc_t rsw = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint8_t*>(w + (int64_t)nt * G * F6_BLOCK), (short)0, G * F6_BLOCK, F6_RSRC_WORD3);
+    // the loads take a fixed lane offset and the group offset as a scalar;
+    // groups past K lie past the resource (zeros, no traffic).
+    const v4u rsa = f6_rsrc(a + (int64_t)mt * G * F6_BLOCK, G * F6_BLOCK);
+    const v4u rsw = f6_rsrc(w + (int64_t)nt * G * F6_BLOCK, G * F6_BLOCK);
     const uint32_t offl = (uint32_t)(3 * wave * 1024 + lane * 16);
-    auto dma = [&](int g, uint8_t* st) {
+    auto dma = [&](int g, int at) {
+        const uint32_t off = g < G ? g * F6_BLOCK : F6_OOR;
+        const uint32_t dst = f6_lds(st) + at + 3 * wave * 1024;
 #pragma unroll
         for (int i = 0; i < 3; ++i) {
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsa, (lds_ptr)(st + (3 * wave + i) * 1024), 16, offl + i * 1024,
-                                                     g * F6_BLOCK, 0, 0);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsw, (lds_ptr)(st + F6_BLOCK + (3 * wave + i) * 1024), 16,
-                                                     offl + i * 1024, g * F6_BLOCK, 0, 0);
+            f6_load_lds(rsa, offl + i * 1024, off, dst + i * 1024);
+            f6_load_lds(rsw, offl + i * 1024, off, dst + F6_BLOCK + i * 1024);
         }
     };
-    // Scales: two windows of 8 groups, [group % 8][sa row 0..127, sw column
-    // 0..127] bf16 (without windows -- scale pointers off a 16-byte boundary
-    // or G not a multiple of 8 -- one slot per group, two groups ahead);
-    // thread t < 128 moves the sa of tile row t, the others the sw of tile
-    // column t-128 (per-channel form: an unused sa).
+    // Scales: two windows of 8 groups, thread t's 16 bytes (8 groups of one
+    // row or column) at t * 16, straight from memory.  Without windows -- scale
+    // pointers off a 16-byte boundary or G not a multiple of 8 -- four slots
+    // of one group, written two groups ahead.  Thread t < 128 moves the sa of
+    // tile row t, the others the sw of tile column t-128 (per-channel form: an
+    // unused sa).
     const bool is_sa = t < F6_BM;
     const uint16_t* s_t = is_sa ? sa + (int64_t)m0 * G : (SG ? sw + (int64_t)n0 * G : sa + (int64_t)m0 * G);
     const uint32_t offs = (uint32_t)(is_sa ? min(t, M - 1 - m0) * G : (SG ? min(t - F6_BM, N - 1 - n0) * G : 0));
-    auto slot = [&](int x) {
-        return WIN ? win + ((x >> 3) & 1) * (F6_WSZ / 2) + (x & 7) * (F6_BM + F6_BN) : win + (x & 1) * (F6_BM + F6_BN);
+    const v4u rss = wave < F6_BM / 64 || !SG ? f6_rsrc(sa + (int64_t)m0 * G, min(F6_BM, M - m0) * G * 2)
+                                             : f6_rsrc(sw + (int64_t)n0 * G, min(F6_BN, N - n0) * G * 2);
+    auto load_win = [&](int wi) {
+        f6_load_lds(rss, offs * 2, wi * 8 < G ? wi * 16 : F6_OOR, f6_lds(win) + (wi & 1) * F6_WSZ + wave * 1024);
     };
-    uint32_t rs;
-    v4u rwin;
-    auto load_win = [&](int wi) { rwin = *reinterpret_cast<const v4u*>(s_t + offs + 8 * wi); };
-    auto store_win = [&](int wi) {
-#pragma unroll
-        for (int gl = 0; gl < 8; ++gl) {
-            const uint32_t h = (rwin[gl >> 1] >> (16 * (gl & 1))) & 0xffffu;
-            slot(wi * 8 + gl)[t] = (uint16_t)h;
-        }
-    };
+    auto slot = [&](int x) { return win + (x & 3) * (F6_BM + F6_BN); };
+    uint32_t rs = 0;
 
     // Operand reads: lane (rc, half) of the 32-row block at tile row b0, k-step s:
     // quarter q = 2 half + s of row b0 + rc, P at q*2048 + row*16, R at
     // 8192 + q*1024 + row*8.
     const int rc = lane & 31, half = lane >> 5;
-    int op[2], orr[2];
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-        const int q = 2 * half + s;
-        op[s] = q * 2048 + rc * 16;
-        orr[s] = F6_R + q * 1024 + rc * 8;
-    }
+    const int opa = 2 * half * 2048 + (wm * 64 + rc) * 16, ora = F6_R + 2 * half * 1024 + (wm * 64 + rc) * 8;
+    const int opw = F6_BLOCK + 2 * half * 2048 + (wn * 64 + rc) * 16;
+    const int orw = F6_BLOCK + F6_R + 2 * half * 1024 + (wn * 64 + rc) * 8;
     float total[2][2][16];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -214,107 +238,134 @@ k2_prefill_f6(const uint8_t* __restrict__ a, const uint8_t* __restrict__ w, cons
             for (int v = 0; v < 16; ++v) total[i][j][v] = 0.0f;
 
     v8i pa[2][2], pw[2][2];
-    v16f acc[2];
-    auto fetch = [&](const uint8_t* st) {
+    auto read = [&](int p, int r, v8i (&dst)[2]) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                const int ra = wm * 64 + i * 32, rw = wn * 64 + i * 32;
-                const v4u a0 = *reinterpret_cast<const v4u*>(st + op[s] + ra * 16);
-                const uint2 a1 = *reinterpret_cast<const uint2*>(st + orr[s] + ra * 8);
-                const v4u w0 = *reinterpret_cast<const v4u*>(st + F6_BLOCK + op[s] + rw * 16);
-                const uint2 w1 = *reinterpret_cast<const uint2*>(st + F6_BLOCK + orr[s] + rw * 8);
-                pa[i][s] = v8i{(int)a0[0], (int)a0[1], (int)a0[2], (int)a0[3], (int)a1.x, (int)a1.y, 0, 0};
-                pw[i][s] = v8i{(int)w0[0], (int)w0[1], (int)w0[2], (int)w0[3], (int)w1.x, (int)w1.y, 0, 0};
-            }
+        for (int s = 0; s < 2; ++s) {
+            const v4u x = *reinterpret_cast<const v4u*>(st + p + s * 2048);
+            const uint2 y = *reinterpret_cast<const uint2*>(st + r + s * 1024);
+            asm volatile("" ::: "memory");  // one 8-byte read each: a merged pair needs copies
+            dst[s] = v8i{(int)x[0], (int)x[1], (int)x[2], (int)x[3], (int)y.x, (int)y.y, 0, 0};
+        }
     };
-    // Blocks in the order (0,0), (0,1), (1,1), (1,0).
-    auto mma = [&](int b) {
-        const int i = b >> 1, j = (b ^ (b >> 1)) & 1;
-        v16f c = {};
-#pragma unroll
-        for (int s = 0; s < 2; ++s)
-            c = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(pa[i][s], pw[j][s], c, F6_FMT, F6_FMT, 0, 127, 0,
-                                                                127);
-        acc[b & 1] = c;
-    };
+    auto read_pa = [&](int at, int i) { read(at + opa + i * 512, at + ora + i * 256, pa[i]); };
+    auto read_pw = [&](int at, int j) { read(at + opw + j * 512, at + orw + j * 256, pw[j]); };
     // Scale products on the matrix cores: a product of two bf16 values has
     // at most 16 significant bits, so sa[m] * sw[n] is exact in fp32 unless
     // it falls below the normal range, and a bf16 MFMA whose only non-zero k
     // term is (sa[row], sw[column]) returns the fp32 product the reference
     // multiplies (sa alone, times bf16 1.0, for per-channel weight scales).
     // Scales whose products reach the fp32 subnormals are in the parity tests
-    // and match the oracle bit for bit.  32x32x16 bf16 operands: lane l
-    // supplies row / column l%32, k = 8(l/32) .. +7, so lanes 32..63 supply
+    // and match the oracle bit for bit.  32x32x8 bf16 operands: lane l
+    // supplies row / column l%32, k = 4(l/32) .. +3, so lanes 32..63 supply
     // zeros; the result has the layout of the fp6 dot.
     const uint32_t keep = half ? 0u : 0xffffu;
-    uint32_t sab[2], swb[2];
-    auto read_scales = [&](const uint16_t* sg) {
+    uint32_t sab[2][2], swb[2][2];
+    auto read_scales = [&](int g, int x) {
+        const uint16_t* sg = WIN ? win + ((g >> 3) & 1) * (F6_WSZ / 2) + (g & 7) : slot(g);
+        constexpr int at = WIN ? 8 : 1;  // elements from one row to the next
 #pragma unroll
-        for (int i = 0; i < 2; ++i) sab[i] = sg[wm * 64 + i * 32 + rc] & keep;
+        for (int i = 0; i < 2; ++i) sab[x][i] = sg[(wm * 64 + i * 32 + rc) * at] & keep;
 #pragma unroll
-        for (int j = 0; j < 2; ++j) swb[j] = (SG ? (uint32_t)sg[F6_BM + wn * 64 + j * 32 + rc] : 0x3f80u) & keep;
+        for (int j = 0; j < 2; ++j)
+            swb[x][j] = (SG ? (uint32_t)sg[(F6_BM + wn * 64 + j * 32 + rc) * at] : 0x3f80u) & keep;
     };
-    v16f prod[2];
-    auto pmma = [&](int b) {
-        const int i = b >> 1, j = (b ^ (b >> 1)) & 1;
-        const v4u av = {sab[i], 0u, 0u, 0u}, bv = {swb[j], 0u, 0u, 0u};
-        prod[b & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, av),
-                                                              __builtin_bit_cast(v8bf, bv), v16f{}, 0, 0, 0);
-    };
-    auto epi = [&](int b) {
-        const int i = b >> 1, j = (b ^ (b >> 1)) & 1;
+    v16f acc[2], prod[2];
+    // fma chain of the block whose dots are in acc[x] (block (i, j) of the
+    // step), outputs [from, to).
+    auto epi = [&](int i, int j, int x, int from, int to) {
 #pragma unroll
-        for (int v = 0; v < 16; ++v) total[i][j][v] = __builtin_fmaf(acc[b & 1][v], prod[b & 1][v], total[i][j][v]);
+        for (int v = from; v < to; ++v) total[i][j][v] = __builtin_fmaf(acc[x][v], prod[x][v], total[i][j][v]);
     };
-    // One group.  The explicit vmcnt(0) completes this wave's direct-to-LDS
-    // loads before the barrier, so after it the whole stage of group g (and,
-    // without windows, the scales of group g) is in LDS and the other stage is
-    // free.  Every LDS read of the step is issued before the next group's
-    // loads, so none of them waits on those.
-    auto step = [&](int g, const uint8_t* st, uint8_t* st_next) {
-        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-        __syncthreads();
-        fetch(st);
-        read_scales(slot(g));
+    // One block: its three MFMAs, each followed by a third of the previous
+    // block's fma chain.  The fences keep that order.
+    auto block = [&](int i, int j, int x, int pi, int pj, int sx) {
+        acc[x] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(pa[i][0], pw[j][0], v16f{}, F6_FMT, F6_FMT, 0, 127,
+                                                                 0, 127);
+        epi(pi, pj, x ^ 1, 0, 5);
         __builtin_amdgcn_sched_barrier(0);
-        if (g + 1 < G) dma(g + 1, st_next);
+        const uint2 av = {sab[sx][i], 0u}, bv = {swb[sx][j], 0u};
+        prod[x] = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(__builtin_bit_cast(v4s, av), __builtin_bit_cast(v4s, bv),
+                                                           v16f{}, 0, 0, 0);
+        epi(pi, pj, x ^ 1, 5, 10);
+        __builtin_amdgcn_sched_barrier(0);
+        acc[x] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(pa[i][1], pw[j][1], acc[x], F6_FMT, F6_FMT, 0, 127,
+                                                                 0, 127);
+        epi(pi, pj, x ^ 1, 10, 16);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // One group.  Blocks (0,c) (0,d) (1,d) (1,c) with c, d alternating between
+    // groups, so each operand is read for the next group right after its last
+    // use and the next group starts on the two read first.  In the middle the
+    // next group's stage is complete (its loads are two groups old) and, past
+    // the barrier, this group's stage is free for the loads of group g + 3.
+    int cur = 0, next = F6_STAGE, far = 2 * F6_STAGE;  // stages of groups g, g + 1, g + 2
+    auto step = [&](int g, auto ORD) {
+        constexpr int c = ORD, d = 1 - ORD, sx = ORD;
+        block(0, c, 0, 1, c ^ 1, sx);  // previous group's last block: (1, its c) = (1, d)
+        block(0, d, 1, 0, c, sx);
+        f6_barrier<6>();
+        dma(g + 3, cur);
         if constexpr (!WIN) {
-            if (g + 1 < G) slot(g + 1)[t] = (uint16_t)rs;
-            if (g + 2 < G) rs = (s_t + g + 2)[offs];
+            slot(g + 2)[t] = (uint16_t)rs;
+            rs = (s_t + min(g + 3, G - 1))[offs];
+            rs = g + 3 < G ? rs : 0u;
         }
+        read_pa(next, 0);
+        read_scales(g + 1, sx ^ 1);
         __builtin_amdgcn_sched_barrier(0);
-        pmma(0);
-        mma(0);
-        pmma(1);
-        mma(1);
-        epi(0);
-        pmma(2);
-        mma(2);
-        epi(1);
-        pmma(3);
-        mma(3);
-        epi(2);
-        epi(3);
-        if constexpr (WIN) {
-            if ((g & 7) == 3 && (g >> 3) + 1 < (G >> 3)) load_win((g >> 3) + 1);
-            if ((g & 7) == 7 && (g >> 3) + 1 < (G >> 3)) store_win((g >> 3) + 1);
-        }
+        block(1, d, 0, 0, d, sx);
+        read_pw(next, d);
+        __builtin_amdgcn_sched_barrier(0);
+        block(1, c, 1, 1, d, sx);
+        read_pw(next, c);
+        read_pa(next, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        const int free = cur;
+        cur = next, next = far, far = free;
     };
 
     if constexpr (WIN) {
         load_win(0);
-        store_win(0);
     } else {
         slot(0)[t] = (s_t + 0)[offs];
-        if (G > 1) rs = (s_t + 1)[offs];
+        const uint32_t s1 = (s_t + min(1, G - 1))[offs], s2 = (s_t + min(2, G - 1))[offs];
+        slot(1)[t] = (uint16_t)(G > 1 ? s1 : 0u);
+        rs = G > 2 ? s2 : 0u;
     }
-    dma(0, st0);
-    for (int g = 0; g < G; g += 2) {
-        step(g, st0, st1);
-        if (g + 1 < G) step(g + 1, st1, st0);
+    dma(0, 0);
+    dma(1, F6_STAGE);
+    dma(2, 2 * F6_STAGE);
+    acc[1] = v16f{};
+    prod[1] = v16f{};
+    f6_barrier<12>();  // the first window and group 0's stage
+    read_pa(0, 0);
+    read_pw(0, 0);
+    read_pw(0, 1);
+    read_pa(0, 1);
+    read_scales(0, 0);
+    using E = std::integral_constant<int, 0>;
+    using O = std::integral_constant<int, 1>;
+    if constexpr (WIN) {
+        for (int g = 0; g < G; g += 8) {
+            step(g, E{});
+            step(g + 1, O{});
+            load_win((g >> 3) + 1);
+            step(g + 2, E{});
+            step(g + 3, O{});
+            step(g + 4, E{});
+            step(g + 5, O{});
+            step(g + 6, E{});
+            step(g + 7, O{});
+        }
+    } else {
+        // A group past K (odd G) has zero dots and scales: the chain stays as it is.
+        for (int g = 0; g < G; g += 2) {
+            step(g, E{});
+            step(g + 1, O{});
+        }
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no load may write LDS after the workgroup has gone
+    epi(1, 1, 1, 0, 16);
 
 #pragma unroll
     for (int j = 0; j < 2; ++j) {

@@ -52,13 +52,12 @@ def use_prefill_path(M, N, K):
     """Prefill-sized GEMMs run on the fp6 matrix cores (``nv4_w4a4_gemm_f6``).
     The operand conversion costs about 1.25 (M + N) K bytes of traffic and one
     launch.  Against the int8 kernels it pays from M = 448 on gate_up (us per
-    call at 383 / 512: 67 int8, 75 fp6 / 89, 80), from M = 704 on weights of
-    4096 x 12288 (512 / 777: 48, 79 / 91, 80), from M = 768 above 4096 x 4096
-    (qkv at 512 / 777: 27, 37 / 42, 42) and from M = 1024 on all of them (o at
-    1024: 34, 34)."""
+    call at 383 / 448 / 512: 63, 80, 89 int8 against 69, 74, 75), from M = 768
+    on the other projections (o at 600 / 777: 25.9, 34.6 against 31.7, 30.7;
+    qkv at 700 / 777: 33.9, 42.0 against 40.9, 40.6; down at 700 / 777: 61.2,
+    85.6 against 65.8, 66.7) and from M = 1024 on smaller weights."""
     nk = N * K
-    return (M >= 1024 or (M >= 768 and nk > 4096 * 4096) or (M >= 704 and nk >= 4096 * 12288)
-            or (M >= 448 and nk >= 4096 * 24576))
+    return M >= 1024 or (M >= 768 and nk >= 4096 * 4096) or (M >= 448 and nk >= 4096 * 24576)
 
 
 def _resolve_path(path, M, N, K):
