@@ -87,4 +87,42 @@ __device__ __forceinline__ v4i unpack8_x16(uint32_t d0, uint32_t d1) {
     return r;
 }
 
+// ---- loads straight into LDS, as volatile asm -------------------------------
+// The compiler would order every later LDS read behind such a load (it tracks
+// few of them apart); with a ring of stages the ones in flight are never the
+// one being read, so the kernel itself waits (lds_ring_barrier) before a stage
+// is read.  Lane l's bytes land at lds + 16 l (4 l); a load past the resource
+// writes zeros.  A kernel that uses them drains vmcnt before it ends.
+constexpr uint32_t kOutOfRange = 0x7fffff00u;  // scalar offset past every resource
+constexpr uint32_t kRsrcWord3 = 0x00020000u;   // buffer resource word 3 (CDNA): 32-bit data format
+
+__device__ __forceinline__ void lds_load16(const v4u& rsrc, uint32_t voff, uint32_t soff, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff),
+                 "s"(rsrc), "s"(soff)
+                 : "memory");
+}
+__device__ __forceinline__ void lds_load4(const v4u& rsrc, uint32_t voff, uint32_t soff, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(lds), "v"(voff),
+                 "s"(rsrc), "s"(soff)
+                 : "memory");
+}
+// A buffer resource in scalar registers (p and bytes are wave-uniform).
+__device__ __forceinline__ v4u scalar_rsrc(const void* p, uint32_t bytes) {
+    const uint64_t x = reinterpret_cast<uint64_t>(p);
+    return v4u{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)x),
+               (uint32_t)__builtin_amdgcn_readfirstlane((int)((x >> 32) & 0xffffu)),
+               (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), kRsrcWord3};
+}
+__device__ __forceinline__ uint32_t lds_address(const void* p) {
+    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
+}
+// All but the wave's N youngest vector-memory loads done and its LDS accesses
+// complete, then the workgroup's barrier.
+template <int N>
+__device__ __forceinline__ void lds_ring_barrier() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
 }  // namespace nv4

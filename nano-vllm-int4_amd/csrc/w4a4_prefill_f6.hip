@@ -55,14 +55,11 @@ constexpr int F6_R = 8192;                              // R part of a block
 constexpr int F6_STAGE = 2 * F6_BLOCK;                  // A block then W block
 constexpr int F6_WSZ = 8 * (F6_BM + F6_BN) * 2;         // 8 groups x (sa[128], sw[128]) bf16
 static_assert(3 * F6_STAGE + 2 * F6_WSZ == 80 * 1024, "80 KiB of LDS: two workgroups per CU");
-constexpr int F6_OOR = 0x7fffff00;                      // scalar offset past every resource
 constexpr int F6_GM = 8;                                // M-tiles per column sweep
-constexpr int F6_RSRC_WORD3 = 0x00020000;               // buffer resource word 3 (CDNA): 32-bit data format
 constexpr int F6_FMT = 3;                               // f8f6f4 operand format: e3m2
 
 typedef short v4s __attribute__((ext_vector_type(4)));
 typedef int v8i __attribute__((ext_vector_type(8)));
-typedef __attribute__((address_space(3))) void* lds_ptr;
 
 // e3m2 codes of the INT4 values: nibble n (two's complement) -> code byte.
 // Four nibbles (one per byte, values 0..15) at a time: two 8-entry byte
@@ -146,32 +143,6 @@ __device__ __forceinline__ void f6_tile(int tm, int tn, int& mt, int& nt) {
     nt = r / gm;
 }
 
-// 16 bytes per lane from a buffer straight into LDS (lane l's at lds + 16 l;
-// out-of-range lanes write zeros), as volatile asm: the compiler would order
-// every later LDS read behind the load (it tracks few of them apart), while
-// here stages in flight are never the ones being read.  The caller waits
-// (vmcnt) and passes a barrier before reading.
-__device__ __forceinline__ void f6_load_lds(const v4u& rsrc, uint32_t voff, uint32_t soff, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff),
-                 "s"(rsrc), "s"(soff)
-                 : "memory");
-}
-__device__ __forceinline__ v4u f6_rsrc(const void* p, uint32_t bytes) {
-    const uint64_t x = reinterpret_cast<uint64_t>(p);
-    return v4u{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)x),
-               (uint32_t)__builtin_amdgcn_readfirstlane((int)((x >> 32) & 0xffffu)),
-               (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), (uint32_t)F6_RSRC_WORD3};
-}
-__device__ __forceinline__ uint32_t f6_lds(const void* p) {
-    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
-}
-template <int N>
-__device__ __forceinline__ void f6_barrier() {  // all but the N youngest loads done, then the workgroup's barrier
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
-
 template <bool SG, bool OF, bool WIN>
 __global__ void __launch_bounds__(F6_T, 2)
 k2_prefill_f6(const uint8_t* __restrict__ a, const uint8_t* __restrict__ w, const uint16_t* __restrict__ sa,
@@ -193,16 +164,16 @@ k2_prefill_f6(const uint8_t* __restrict__ a, const uint8_t* __restrict__ w, cons
     // the 16 bytes at l * 16.  Buffer resources over the tile's G blocks, so
     // the loads take a fixed lane offset and the group offset as a scalar;
     // groups past K lie past the resource (zeros, no traffic).
-    const v4u rsa = f6_rsrc(a + (int64_t)mt * G * F6_BLOCK, G * F6_BLOCK);
-    const v4u rsw = f6_rsrc(w + (int64_t)nt * G * F6_BLOCK, G * F6_BLOCK);
+    const v4u rsa = scalar_rsrc(a + (int64_t)mt * G * F6_BLOCK, G * F6_BLOCK);
+    const v4u rsw = scalar_rsrc(w + (int64_t)nt * G * F6_BLOCK, G * F6_BLOCK);
     const uint32_t offl = (uint32_t)(3 * wave * 1024 + lane * 16);
     auto dma = [&](int g, int at) {
-        const uint32_t off = g < G ? g * F6_BLOCK : F6_OOR;
-        const uint32_t dst = f6_lds(st) + at + 3 * wave * 1024;
+        const uint32_t off = g < G ? g * F6_BLOCK : kOutOfRange;
+        const uint32_t dst = lds_address(st) + at + 3 * wave * 1024;
 #pragma unroll
         for (int i = 0; i < 3; ++i) {
-            f6_load_lds(rsa, offl + i * 1024, off, dst + i * 1024);
-            f6_load_lds(rsw, offl + i * 1024, off, dst + F6_BLOCK + i * 1024);
+            lds_load16(rsa, offl + i * 1024, off, dst + i * 1024);
+            lds_load16(rsw, offl + i * 1024, off, dst + F6_BLOCK + i * 1024);
         }
     };
     // Scales: two windows of 8 groups, thread t's 16 bytes (8 groups of one
@@ -214,10 +185,10 @@ k2_prefill_f6(const uint8_t* __restrict__ a, const uint8_t* __restrict__ w, cons
     const bool is_sa = t < F6_BM;
     const uint16_t* s_t = is_sa ? sa + (int64_t)m0 * G : (SG ? sw + (int64_t)n0 * G : sa + (int64_t)m0 * G);
     const uint32_t offs = (uint32_t)(is_sa ? min(t, M - 1 - m0) * G : (SG ? min(t - F6_BM, N - 1 - n0) * G : 0));
-    const v4u rss = wave < F6_BM / 64 || !SG ? f6_rsrc(sa + (int64_t)m0 * G, min(F6_BM, M - m0) * G * 2)
-                                             : f6_rsrc(sw + (int64_t)n0 * G, min(F6_BN, N - n0) * G * 2);
+    const v4u rss = wave < F6_BM / 64 || !SG ? scalar_rsrc(sa + (int64_t)m0 * G, min(F6_BM, M - m0) * G * 2)
+                                             : scalar_rsrc(sw + (int64_t)n0 * G, min(F6_BN, N - n0) * G * 2);
     auto load_win = [&](int wi) {
-        f6_load_lds(rss, offs * 2, wi * 8 < G ? wi * 16 : F6_OOR, f6_lds(win) + (wi & 1) * F6_WSZ + wave * 1024);
+        lds_load16(rss, offs * 2, wi * 8 < G ? wi * 16 : kOutOfRange, lds_address(win) + (wi & 1) * F6_WSZ + wave * 1024);
     };
     auto slot = [&](int x) { return win + (x & 3) * (F6_BM + F6_BN); };
     uint32_t rs = 0;
@@ -303,7 +274,7 @@ k2_prefill_f6(const uint8_t* __restrict__ a, const uint8_t* __restrict__ w, cons
         constexpr int c = ORD, d = 1 - ORD, sx = ORD;
         block(0, c, 0, 1, c ^ 1, sx);  // previous group's last block: (1, its c) = (1, d)
         block(0, d, 1, 0, c, sx);
-        f6_barrier<6>();
+        lds_ring_barrier<6>();
         dma(g + 3, cur);
         if constexpr (!WIN) {
             slot(g + 2)[t] = (uint16_t)rs;
@@ -337,7 +308,7 @@ k2_prefill_f6(const uint8_t* __restrict__ a, const uint8_t* __restrict__ w, cons
     dma(2, 2 * F6_STAGE);
     acc[1] = v16f{};
     prod[1] = v16f{};
-    f6_barrier<12>();  // the first window and group 0's stage
+    lds_ring_barrier<12>();  // the first window and group 0's stage
     read_pa(0, 0);
     read_pw(0, 0);
     read_pw(0, 1);

@@ -19,8 +19,12 @@ which at 17..32 rows costs more than splitting K when K is long or the
 workgroups are several per CU) take the split-K form
 (``nv4_w4a16_gemm_ws``): 64-column workgroups per 1024-deep K slice writing
 fp32 partials into a workspace from torch's caching allocator, added in slice
-order by a second launch.  Both are deterministic and graph-capturable.  At prefill sizes (M > 64) the weight is dequantized once
-into a dense [K, N] tensor (``nv4_w4a16_dequant``, the same per-element
+order by a second launch.  Both are deterministic and graph-capturable.
+
+65 to 768 rows (``mid_form``) run ``nv4_w4a16_gemm_mid``: the codes meet
+reordered activations on the 32 x 32 matrix cores, no dense weight in between.
+Beyond that the weight is
+dequantized once into a dense [K, N] tensor (``nv4_w4a16_dequant``, the same per-element
 rounding) and the product runs as a library GEMM (torch.mm on hipBLASLt,
 fp32 accumulation).
 """
@@ -80,6 +84,16 @@ def one_launch(M, N, K, device=None):
     return K <= 4096 and (N + 31) // 32 <= _CUS[idx]
 
 
+def mid_form(M):
+    """Whether ``nv4_w4a16_gemm_mid`` serves M rows.  Against the dense weight
+    and the library's product it wins up to 512 rows on every projection (us
+    per call: o 38 / 43, qkv 47 / 62, down 93 / 107, gate_up 114 / 134) and
+    breaks even around 1024 (52 / 53, 70 / 74, 132 / 131, 214 / 220).  Up to 64
+    rows the results must not depend on N (fused projections equal the separate
+    ones bit for bit), which its K slices do."""
+    return 64 < M <= 768
+
+
 def dequant_matmul_w4a16(x, qweight, qzeros, scales, group_size=128, out=None):
     """x [M,K] bf16/fp16 -> out [M,N] in x's dtype."""
     if x.ndim != 2 or x.dtype not in _DT:
@@ -109,6 +123,14 @@ def dequant_matmul_w4a16(x, qweight, qzeros, scales, group_size=128, out=None):
                                     ctypes.c_void_p(qweight.data_ptr()), ctypes.c_void_p(qzeros.data_ptr()),
                                     ctypes.c_void_p(scales.data_ptr()), ctypes.c_void_p(out.data_ptr()),
                                     _DT[out.dtype], M, N, K, group_size, ctypes.c_void_p(stream))
+        elif (mid_form(M) and (nbytes := lib.nv4_w4a16_gemm_mid_workspace(M, N, K)) > 0
+              and not any(t.data_ptr() % 16 for t in (x, qweight, scales, out))):
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+            rc = lib.nv4_w4a16_gemm_mid(ctypes.c_void_p(x.data_ptr()), _DT[x.dtype],
+                                        ctypes.c_void_p(qweight.data_ptr()), ctypes.c_void_p(qzeros.data_ptr()),
+                                        ctypes.c_void_p(scales.data_ptr()), ctypes.c_void_p(out.data_ptr()),
+                                        _DT[out.dtype], ctypes.c_void_p(ws.data_ptr()), nbytes, M, N, K, group_size,
+                                        ctypes.c_void_p(stream))
         elif M <= 64:
             S = (K + SLICE_K - 1) // SLICE_K
             ws = torch.empty((S * M * N,), dtype=torch.float32, device=x.device)
