@@ -311,6 +311,10 @@ int nv4_w4a16_gemm(const void* x, int x_dtype, const int32_t* qweight, const int
                    const void* scales, void* out, int out_dtype,
                    int64_t M, int64_t N, int64_t K, int group, void* stream);
 
+/* Whether nv4_w4a16_gemm runs these sizes in its one-launch decode kernel on
+ * the current device (1) or in its general one (0). */
+int nv4_w4a16_one_launch(int64_t M, int64_t N, int64_t K);
+
 /*
  * nv4_w4a16_gemm with a caller-provided fp32 workspace, for decode sizes
  * (M <= 64; larger M runs nv4_w4a16_gemm and ignores the workspace): K is

@@ -806,6 +806,10 @@ extern "C" int nv4_w4a16_dequant(const int32_t* qweight, const int32_t* qzeros, 
     return (int)hipGetLastError();
 }
 
+extern "C" int nv4_w4a16_one_launch(int64_t M, int64_t N, int64_t K) {
+    return M >= 1 && N >= 1 && K >= 1 && nv4::one_launch_fits(M, N, K);
+}
+
 extern "C" int nv4_w4a16_gemm(const void* x, int x_dtype, const int32_t* qweight, const int32_t* qzeros,
                               const void* scales, void* out, int out_dtype,
                               int64_t M, int64_t N, int64_t K, int group, void* stream) {

@@ -53,6 +53,7 @@ SIGNATURES = {
     "nv4_w4a4_tile_weights": ([_P, _P, _I64, _I64, _P], _I),
     "nv4_w4a4_untile_weights": ([_P, _P, _I64, _I64, _P], _I),
     "nv4_w4a16_gemm": ([_P, _I, _P, _P, _P, _P, _I, _I64, _I64, _I64, _I, _P], _I),
+    "nv4_w4a16_one_launch": ([_I64, _I64, _I64], _I),
     "nv4_w4a16_gemm_ws": ([_P, _I, _P, _P, _P, _P, _I, _P, _I64, _I64, _I64, _I64, _I, _P], _I),
     "nv4_w4a16_gemm_mid_workspace": ([_I64, _I64, _I64], _I64),
     "nv4_w4a16_gemm_mid": ([_P, _I, _P, _P, _P, _P, _I, _P, _I64, _I64, _I64, _I64, _I, _P], _I),
@@ -83,7 +84,12 @@ SIGNATURES = {
 }
 
 _lib = None
+_native = None
 _lock = threading.Lock()
+
+# What nv4._ops calls, in the order of its entry-point table.
+_OPS_ENTRIES = ("nv4_w4a4_linear", "nv4_w4a4_linear_tiled", "nv4_w4a4_linear_rowtiled", "nv4_w4a16_gemm",
+                "nv4_w4a16_gemm_ws", "nv4_w4a16_gemm_mid", "nv4_w4a16_gemm_mid_workspace", "nv4_w4a16_one_launch")
 
 
 class NV4LibraryError(RuntimeError):
@@ -111,6 +117,22 @@ def load():
                 fn.restype = res
             _lib = lib
     return _lib
+
+
+def ops():
+    """nv4._ops, the native per-call path of the linear operators, bound to the
+    loaded library; raise NV4LibraryError when it is not built."""
+    global _native
+    if _native is None:
+        lib = load()
+        try:
+            from . import _ops
+        except ImportError as exc:
+            raise NV4LibraryError("nv4/_ops.so is missing or does not load: build it first "
+                                  f"(make -C nano-vllm-int4_amd, or __graft_entry__.build()): {exc}") from exc
+        _ops.bind(tuple(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in _OPS_ENTRIES))
+        _native = _ops
+    return _native
 
 
 def strerror(code: int) -> str:

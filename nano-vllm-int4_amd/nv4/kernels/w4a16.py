@@ -38,7 +38,7 @@ from .. import _lib
 
 _DT = {torch.bfloat16: _lib.BF16, torch.float16: _lib.FP16}
 SLICE_K = 1024  # K per partial of the decode-size split
-ONE_LAUNCH_MAX_M = 32  # nv4_w4a16_gemm runs one launch up to this M (see one_launch)
+SPLIT_MAX_M, MID_MAX_M = 64, 768  # largest M of nv4_w4a16_gemm_ws and (see mid_form) of nv4_w4a16_gemm_mid
 
 
 def dequant_w4a16(qweight, qzeros, scales, dtype=torch.bfloat16, group_size=128):
@@ -66,22 +66,14 @@ def dequant_w4a16(qweight, qzeros, scales, dtype=torch.bfloat16, group_size=128)
     return w
 
 
-_CUS = {}
-
-
 def one_launch(M, N, K, device=None):
-    """Whether ``nv4_w4a16_gemm`` runs these sizes in its one-launch kernel
-    (the rule it applies itself): the packed weight (K * N / 2 bytes) under
-    2 GiB and M <= 16, or M <= 32 with K <= 4096 and ceil(N / 32) workgroups
-    at most one per CU."""
-    if M > ONE_LAUNCH_MAX_M or K * N // 2 >= (1 << 31):
-        return False
-    if M <= 16:
-        return True
-    idx = (torch.device(device).index or 0) if device is not None else torch.cuda.current_device()
-    if idx not in _CUS:
-        _CUS[idx] = torch.cuda.get_device_properties(idx).multi_processor_count
-    return K <= 4096 and (N + 31) // 32 <= _CUS[idx]
+    """Whether ``nv4_w4a16_gemm`` runs these sizes in its one-launch kernel: the
+    packed weight (K * N / 2 bytes) under 2 GiB and M <= 16, or M <= 32 with K <=
+    4096 and ceil(N / 32) workgroups at most one per CU of ``device``."""
+    if device is None:
+        return bool(_lib.load().nv4_w4a16_one_launch(M, N, K))
+    with torch.cuda.device(device):
+        return bool(_lib.load().nv4_w4a16_one_launch(M, N, K))
 
 
 def mid_form(M):
@@ -91,11 +83,16 @@ def mid_form(M):
     breaks even around 1024 (52 / 53, 70 / 74, 132 / 131, 214 / 220).  Up to 64
     rows the results must not depend on N (fused projections equal the separate
     ones bit for bit), which its K slices do."""
-    return 64 < M <= 768
+    return SPLIT_MAX_M < M <= MID_MAX_M
 
 
 def dequant_matmul_w4a16(x, qweight, qzeros, scales, group_size=128, out=None):
     """x [M,K] bf16/fp16 -> out [M,N] in x's dtype."""
+    if out is None and group_size == 128 and x.is_cuda:
+        # The plain call, natively; None when it is not one (or has more rows).
+        native = _lib.ops().dequant_matmul_w4a16(x, qweight, qzeros, scales, SPLIT_MAX_M, SLICE_K, MID_MAX_M)
+        if native is not None:
+            return native
     if x.ndim != 2 or x.dtype not in _DT:
         raise ValueError("Expected BF16 or FP16 activations [M,K]")
     M, K = x.shape
@@ -118,7 +115,7 @@ def dequant_matmul_w4a16(x, qweight, qzeros, scales, group_size=128, out=None):
     lib = _lib.load()
     stream = torch.cuda.current_stream(x.device).cuda_stream
     with torch.cuda.device(x.device):
-        if one_launch(M, N, K, x.device):
+        if one_launch(M, N, K):
             rc = lib.nv4_w4a16_gemm(ctypes.c_void_p(x.data_ptr()), _DT[x.dtype],
                                     ctypes.c_void_p(qweight.data_ptr()), ctypes.c_void_p(qzeros.data_ptr()),
                                     ctypes.c_void_p(scales.data_ptr()), ctypes.c_void_p(out.data_ptr()),
@@ -131,7 +128,7 @@ def dequant_matmul_w4a16(x, qweight, qzeros, scales, group_size=128, out=None):
                                         ctypes.c_void_p(scales.data_ptr()), ctypes.c_void_p(out.data_ptr()),
                                         _DT[out.dtype], ctypes.c_void_p(ws.data_ptr()), nbytes, M, N, K, group_size,
                                         ctypes.c_void_p(stream))
-        elif M <= 64:
+        elif M <= SPLIT_MAX_M:
             S = (K + SLICE_K - 1) // SLICE_K
             ws = torch.empty((S * M * N,), dtype=torch.float32, device=x.device)
             rc = lib.nv4_w4a16_gemm_ws(ctypes.c_void_p(x.data_ptr()), _DT[x.dtype],

@@ -48,6 +48,10 @@ def _validate_config(cfg: GroupedConfig) -> None:
 PATHS = ("int8", "fp8", "fp6")
 
 
+# No size below this M runs on the fp6 matrix cores (``use_prefill_path``).
+PREFILL_MIN_M = 448
+
+
 def use_prefill_path(M, N, K):
     """Prefill-sized GEMMs run on the fp6 matrix cores (``nv4_w4a4_gemm_f6``).
     The operand conversion costs about 1.25 (M + N) K bytes of traffic and one
@@ -57,7 +61,7 @@ def use_prefill_path(M, N, K):
     qkv at 700 / 777: 33.9, 42.0 against 40.9, 40.6; down at 700 / 777: 61.2,
     85.6 against 65.8, 66.7) and from M = 1024 on smaller weights."""
     nk = N * K
-    return M >= 1024 or (M >= 768 and nk >= 4096 * 4096) or (M >= 448 and nk >= 4096 * 24576)
+    return M >= 1024 or (M >= 768 and nk >= 4096 * 4096) or (M >= PREFILL_MIN_M and nk >= 4096 * 24576)
 
 
 def _resolve_path(path, M, N, K):

@@ -20,7 +20,7 @@ import torch
 
 from .. import _lib
 from .rht_a4 import rht_quant_pack, rowtiled_rows
-from .w4a4_grouped import ROWTILED_MAX_M, _check_weights_f6, _launch, use_prefill_path
+from .w4a4_grouped import PREFILL_MIN_M, ROWTILED_MAX_M, _check_weights_f6, _launch, use_prefill_path
 
 
 def w4a4_linear(x, signs, w_packed, w_scale, *, out=None, out_packed=None, out_scale=None, weights_tiled=False,
@@ -32,6 +32,12 @@ def w4a4_linear(x, signs, w_packed, w_scale, *, out=None, out_packed=None, out_s
     ``packed_rowtiled``: whether ``out_packed`` receives the codes in the
     row-tiled order ([ceil(M/16)*16, K/2]; tiled weights, M <= 32); None
     chooses it exactly when ``out_packed`` is not given."""
+    if out is None and out_packed is None and out_scale is None and weights_f6 is None and packed_rowtiled is None \
+            and x.is_cuda:
+        # The plain call below the fp6 sizes, natively; None when it is not one.
+        native = _lib.ops().w4a4_linear(x, signs, w_packed, w_scale, weights_tiled, ROWTILED_MAX_M, PREFILL_MIN_M)
+        if native is not None:
+            return native
     if x.ndim != 2 or x.dtype != torch.bfloat16 or x.shape[1] not in (4096, 12288) or x.shape[0] < 1:
         raise ValueError("Expected BF16 X[M,K], M>0, K=4096/12288")
     M, K = x.shape

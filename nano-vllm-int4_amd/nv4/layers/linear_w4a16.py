@@ -45,13 +45,14 @@ class W4A16Linear(nn.Module):
                                    requires_grad=False)
 
     def forward(self, x):
-        shape = x.shape
-        x = x.reshape(-1, self.in_features).contiguous()
         # (after fuse_w4a16 the parameters are column views of the fused
         # tensors; a direct call then reads contiguous copies)
-        out = dequant_matmul_w4a16(x, self.qweight.contiguous(), self.qzeros.contiguous(), self.scales.contiguous(),
-                                   self.group_size)
-        return out.reshape(*shape[:-1], self.out_features)
+        p = self._parameters
+        weights = [p[name].contiguous() for name in ("qweight", "qzeros", "scales")]
+        if x.ndim == 2 and x.shape[1] == self.in_features and x.is_contiguous():
+            return dequant_matmul_w4a16(x, *weights, self.group_size)
+        out = dequant_matmul_w4a16(x.reshape(-1, self.in_features).contiguous(), *weights, self.group_size)
+        return out.reshape(*x.shape[:-1], self.out_features)
 
 
 @torch.no_grad()

@@ -32,8 +32,8 @@ from torch import nn
 import torch.distributed as dist
 
 from .. import _lib
-from ..kernels.w4a4_grouped import (ROWTILED_MAX_M, keep_weights_f6, rowtiled_silu_fits, tile_weights, untile_weights,
-                                   w4a4_gemm_rowtiled, w4a4_gemm_rowtiled_silu, w4a4_grouped_gemm, weights_to_f6)
+from ..kernels.w4a4_grouped import (PREFILL_MIN_M, ROWTILED_MAX_M, keep_weights_f6, rowtiled_silu_fits,
+                                   tile_weights, untile_weights, w4a4_gemm_rowtiled, w4a4_gemm_rowtiled_silu, w4a4_grouped_gemm, weights_to_f6)
 from ..kernels.w4a4_linear import w4a4_linear
 
 
@@ -130,11 +130,17 @@ class W4A4Linear(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if x.shape[-1] != self.in_features or x.dtype != torch.bfloat16:
             raise ValueError("W4A4Linear requires BF16 activations with the configured input width")
-        flat = x.reshape(-1, self.in_features).contiguous()
         # RHT + quantize + pack, then the grouped INT4 GEMM; packed codes and
         # scales come from the caching allocator, so the forward can be
-        # captured in a HIP graph.
-        out = w4a4_linear(flat, self.signs, self.packed_weight, self.weight_scale, weights_tiled=self.weights_tiled,
+        # captured in a HIP graph.  (Buffers by dict: nn.Module's attribute
+        # lookup costs more than the checks.)
+        b = self._buffers
+        if x.ndim == 2 and x.is_contiguous():
+            f6 = self._f6() if b["weight_f6"] is not None and x.shape[0] >= PREFILL_MIN_M else None
+            return w4a4_linear(x, b["signs"], b["packed_weight"], b["weight_scale"], weights_tiled=self.weights_tiled,
+                               weights_f6=f6)
+        flat = x.reshape(-1, self.in_features).contiguous()
+        out = w4a4_linear(flat, b["signs"], b["packed_weight"], b["weight_scale"], weights_tiled=self.weights_tiled,
                           weights_f6=self._f6())
         return out.reshape(*x.shape[:-1], self.out_features)
 
