@@ -32,8 +32,9 @@
 //    Loads run several rounds ahead.
 //  * k2_wide (M <= 32, wide N): waves own column blocks over the whole K,
 //    activations widened once per CU into LDS.
-//  * k2_mid (M > 32, w4a4_mid.hip): 32..48 x 64..128 tiles, whole K per wave.
-//  * k2_prefill (M >= 2048, w4a4_prefill.hip): LDS-staged 128x128 tiles.
+//  * k2_mid, k2_mid32 (M > 32, w4a4_mid.hip): 32..64 x 64..128 tiles, whole K
+//    per wave.
+//  * k2_prefill (M >= 3072, w4a4_prefill.hip): LDS-staged 128x128 tiles.
 #include "k2_launch.h"
 #include "norm_ops.h"
 #include "nv4_common.h"
@@ -735,10 +736,11 @@ hipError_t dispatch(const int8_t* a, const int8_t* w, const void* sa, const void
     if (M <= 64 && (int64_t)((M + 15) / 16) * ((N + 15) / 16) <= 5LL * device_cu_count())
         return M <= 48 ? launch_dec<3, TW, false, SG, OF>(a, w, sa, sw, out, M, N, K, st)
                        : launch_dec<4, TW, false, SG, OF>(a, w, sa, sw, out, M, N, K, st);
-    // From M = 2048 the 128 x 128 tiles fill the chip and move fewer bytes (o /
-    // qkv / down / gate_up at 2048: 59 / 93 / 167 / 317 us against 65 / 95 /
-    // 172 / 326; at 1024 46 / 59 / 125 / 169 against 34 / 49 / 89 / 163).
-    if (M < 2048) return k2_mid_launch(a, w, sa, sw, SG, out, OF, TW, M, N, K, st);
+    // At M = 4096 the 128 x 128 tiles fill the chip and move fewer bytes (gate_up
+    // 613 us against 637, qkv 164 / 166, down 316 / 309, o 114 / 111); at 2048 the
+    // smaller ones still win or tie (o / qkv / down / gate_up: 54 / 88 / 150 / 317
+    // against 59 / 93 / 167 / 317).
+    if (M < 3072) return k2_mid_launch(a, w, sa, sw, SG, out, OF, TW, M, N, K, st);
     return k2_prefill_launch(a, w, sa, sw, SG, out, OF, TW, M, N, K, st);
 }
 

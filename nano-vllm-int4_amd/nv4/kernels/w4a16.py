@@ -21,7 +21,7 @@ workgroups are several per CU) take the split-K form
 fp32 partials into a workspace from torch's caching allocator, added in slice
 order by a second launch.  Both are deterministic and graph-capturable.
 
-65 to 768 rows (``mid_form``) run ``nv4_w4a16_gemm_mid``: the codes meet
+65 to 640 rows (``mid_form``) run ``nv4_w4a16_gemm_mid``: the codes meet
 reordered activations on the 32 x 32 matrix cores, no dense weight in between.
 Beyond that the weight is
 dequantized once into a dense [K, N] tensor (``nv4_w4a16_dequant``, the same per-element
@@ -38,7 +38,7 @@ from .. import _lib
 
 _DT = {torch.bfloat16: _lib.BF16, torch.float16: _lib.FP16}
 SLICE_K = 1024  # K per partial of the decode-size split
-SPLIT_MAX_M, MID_MAX_M = 64, 768  # largest M of nv4_w4a16_gemm_ws and (see mid_form) of nv4_w4a16_gemm_mid
+SPLIT_MAX_M, MID_MAX_M = 64, 640  # largest M of nv4_w4a16_gemm_ws and (see mid_form) of nv4_w4a16_gemm_mid
 
 
 def dequant_w4a16(qweight, qzeros, scales, dtype=torch.bfloat16, group_size=128):
@@ -78,11 +78,11 @@ def one_launch(M, N, K, device=None):
 
 def mid_form(M):
     """Whether ``nv4_w4a16_gemm_mid`` serves M rows.  Against the dense weight
-    and the library's product it wins up to 512 rows on every projection (us
-    per call: o 38 / 43, qkv 47 / 62, down 93 / 107, gate_up 114 / 134) and
-    breaks even around 1024 (52 / 53, 70 / 74, 132 / 131, 214 / 220).  Up to 64
-    rows the results must not depend on N (fused projections equal the separate
-    ones bit for bit), which its K slices do."""
+    and the library's product it wins on every projection up to 640 rows (us
+    per call at 300 / 640: o 31, 48 against 48, 51; qkv 35, 57 / 45, 59; down 54,
+    121 / 119, 126; gate_up 77, 154 / 113, 175) and loses on qkv at 768 (71 / 63).
+    Up to 64 rows the results must not depend on N (fused projections equal the
+    separate ones bit for bit), which its K slices do."""
     return SPLIT_MAX_M < M <= MID_MAX_M
 
 

@@ -56,12 +56,12 @@ def use_prefill_path(M, N, K):
     """Prefill-sized GEMMs run on the fp6 matrix cores (``nv4_w4a4_gemm_f6``).
     The operand conversion costs about 1.25 (M + N) K bytes of traffic and one
     launch.  Against the int8 kernels it pays from M = 448 on gate_up (us per
-    call at 383 / 448 / 512: 63, 80, 89 int8 against 69, 74, 75), from M = 768
-    on the other projections (o at 600 / 777: 25.9, 34.6 against 31.7, 30.7;
-    qkv at 700 / 777: 33.9, 42.0 against 40.9, 40.6; down at 700 / 777: 61.2,
-    85.6 against 65.8, 66.7) and from M = 1024 on smaller weights."""
+    call at 383 / 448 / 512: 65, 77, 81 int8 against 72, 74, 78), from M = 768
+    on the narrower projections above 4096 x 4096 (qkv at 700 / 777: 36, 43
+    against 42, 42; down at 700 / 832: 65, 71 against 67, 69) and past M = 1024
+    on all others (o at 777 / 1024: 30.5, 31.7 against 32.4, 31.7)."""
     nk = N * K
-    return M >= 1024 or (M >= 768 and nk >= 4096 * 4096) or (M >= PREFILL_MIN_M and nk >= 4096 * 24576)
+    return M > 1024 or (M >= 768 and nk > 4096 * 4096) or (M >= PREFILL_MIN_M and nk >= 4096 * 24576)
 
 
 def _resolve_path(path, M, N, K):

@@ -1,7 +1,7 @@
-"""GPU parity of the mid-sized grouped W4A4 GEMM (``k2_mid``, 32 < M < 2048).
+"""GPU parity of the mid-sized grouped W4A4 GEMM (``k2_mid``, ``k2_mid32``, 32 < M < 3072).
 
 Bit for bit against the oracle (benchmarks/verify_w4a4_aw_grouped.py:13-29) at
-the edges of its tiles (32 and 48 rows, 64 and 128 columns), of the range its
+the edges of its tiles (32, 48 and 64 rows, 64 and 128 columns), of the range its
 dispatch gives it, and of the two sequences it runs: scales inside the range
 of the folded 2^-8, and the literal one for scales outside, K / 128 not a
 multiple of 8, or scale pointers off a 16-byte boundary.
@@ -41,11 +41,11 @@ def check(M, N, K, ap, wp, sa, sw, unaligned=False):
     assert_bits_equal(out32.cpu().numpy().view(np.uint32), exp32.view(np.uint32), "fp32")
 
 
-# On 256 CUs: 32 x 64 tiles (the first five), 32 x 128 (200 x 4096, one round),
-# 48 x 128 (33 and 96 x 24576; 97 ends 47 rows into its third tile).
+# On 256 CUs: 32 x 64 tiles (the first five and the last two), 32 x 128 (200 x
+# 4096), 48 x 128 (33 x 24576), 64 x 128 (97 x 24584, 450 x 8184).
 @pytest.mark.parametrize("M,N,K", [(65, 8, 1024), (65, 72, 1024), (97, 200, 2048), (64, 6144, 1024), (129, 1040, 4096),
-                                   (200, 4096, 1024), (33, 24576, 1024), (97, 24584, 1024), (70, 136, 12288),
-                                   (2047, 136, 1024)])
+                                   (200, 4096, 1024), (33, 24576, 1024), (97, 24584, 1024), (450, 8184, 1024),
+                                   (70, 136, 12288), (2047, 136, 1024)])
 @pytest.mark.parametrize("grouped", [True, False])
 def test_tiles(M, N, K, grouped):
     ap, wp, sa, sw = gemm_inputs(M, N, K, M + 3 * N + K)
@@ -59,9 +59,9 @@ def test_literal_by_shape(M, N, K, unaligned):
     check(M, N, K, ap, wp, sa, sw, unaligned)
 
 
-# The last one: the 128 x 128 tiles that take over at M = 2048.
+# The last one: the 128 x 128 tiles that take over at M = 3072.
 @pytest.mark.parametrize("M,N,K,rows", [(100, 200, 1024, True), (100, 200, 1024, False), (200, 4096, 1024, True),
-                                        (100, 24576, 1024, False), (2050, 136, 1024, True)])
+                                        (33, 24576, 1024, False), (450, 8184, 1024, True), (3080, 136, 1024, True)])
 def test_scales_outside_the_fold(M, N, K, rows):
     """One tile row (or column panel) leaves the range; its neighbours do not."""
     ap, wp, sa, sw = gemm_inputs(M, N, K, M + N + K + 1)
