@@ -15,6 +15,7 @@
 // fp32 partial tiles are added in LDS in wave order at the end (fixed
 // order, deterministic).  Each lane's B operand is exactly one qweight word
 // (8 consecutive k of one column), dequantized in registers.
+#include "k3_codes.h"
 #include "k3_reduce.h"
 #include "nv4_common.h"
 
@@ -198,138 +199,179 @@ k3_w4a16(const uint16_t* __restrict__ x, const int32_t* __restrict__ qweight,
 //    32-k step, and all of the slice's loads (8 per lane) are issued up
 //    front; the four words feed four MFMAs whose output columns are
 //    4c + j (j = word);
-//  * activations: the slice's rows (ROWS x 1024 bf16) are copied into LDS in
-//    whole lines once per workgroup and read back as MFMA A operands
-//    (16-byte chunks XOR-swizzled by row);
-//  * dequantization (W16Traits::dequant8): two byte permutes put a word's
-//    nibbles in k order as bytes; bf16 takes fma(q, s, -(z+1) s) (exact in
-//    fp32) and rounds once per value, fp16 builds each half as 1024 + q
-//    (bit pattern 0x6400 | q) and rounds (q - z - 1) * s once with packed
-//    fp16 arithmetic -- the reference's rounding of the dequantized weight;
-//  * wave w takes the 8 consecutive 32-k steps 8w .. 8w+7 of the slice (two
-//    groups, so two scale/zero preparations per column); the four waves'
-//    fp32 tiles are added in wave order in LDS, and the slice's [M, N] fp32
-//    partial goes to the workspace; a second kernel adds the slices in order
-//    and rounds once (no atomics, same bits on every run).
+//  * activations: the slice goes through LDS in two halves of 512 k, copied in
+//    whole lines and read back as MFMA A operands (16-byte octets XOR-swizzled
+//    by row, in the order in which a word's codes come out), so that two
+//    workgroups share a CU and one computes while the other loads;
+//  * dequantization per group (k3_codes.h): wave w takes group w of each half,
+//    four steps of biased codes and an all-ones MFMA for the rows' sums, then
+//    two fmas per output; rows with huge magnitudes run on unbiased codes;
+//  * the four waves' fp32 tiles are added in wave order in LDS, and the slice's
+//    [M, N] fp32 partial goes to the workspace; a second kernel adds the slices
+//    in order and rounds once (no atomics, same bits on every run, and for each
+//    column the same whatever N is).
+// Bound: 33..64 rows by the dequantizing VALU beside the MFMAs (a word's eight
+// codes cost 8 operations; scaling and rounding each weight cost about 24),
+// below that by the weight stream.  us with both launches, cold weights,
+// against a whole-slice form that scaled each weight: [6144 x 4096] 45 rows
+// 16.8 -> 14.3, 64 rows 19.8 -> 17.9; [24576 x 4096] 17 rows 24.2 -> 21.6,
+// 45 rows 41.9 -> 31.5, 64 rows 49.4 -> 39.7; [4096 x 12288] 45 rows 24.5 ->
+// 20.1, 64 rows 28.1 -> 24.6; [4096 x 4096] unchanged.  The distance to the
+// 64-bit product falls too, bf16 2.3e-3 -> 1.7e-3 (the rounding of the result).
 // ----------------------------------------------------------------------------
+// An activation octet x0..x7 (16-bit pairs) reordered to x0 x4 x1 x5 x2 x6 x3 x7.
+__device__ __forceinline__ v4u octet_order(v4u v) {
+    return v4u{__builtin_amdgcn_perm(v[2], v[0], 0x05040100u), __builtin_amdgcn_perm(v[2], v[0], 0x07060302u),
+               __builtin_amdgcn_perm(v[3], v[1], 0x05040100u), __builtin_amdgcn_perm(v[3], v[1], 0x07060302u)};
+}
+
 constexpr int K3_KS = 1024;  // k per slice
 constexpr int K3_RSRC_WORD3 = 0x00020000;  // buffer resource word 3 (CDNA): 32-bit data format
 constexpr int K3_NB = 64;    // columns per workgroup
 
-__device__ __forceinline__ int k3_swz(int r, int c) { return r * (K3_KS * 2) + ((c ^ (r & 7)) << 4); }
 
-template <int MB, bool XF16>
-__global__ void __launch_bounds__(256, 1)
+// PASS: passes over the activations in LDS, 1 (the whole slice) or 2 (halves).
+template <int MB, bool XF16, int PASS>
+__global__ void __launch_bounds__(256, PASS)
 k3_dec(const uint16_t* __restrict__ x, const int32_t* __restrict__ qweight, const int32_t* __restrict__ qzeros,
        const uint16_t* __restrict__ scales, float* __restrict__ ws, int M, int N, int K) {
-    using TR = W16Traits<XF16>;
+    using MC = MidCode<XF16>;
+    using vec = typename MC::vec;
     constexpr int ROWS = MB * 16;
-    __shared__ __align__(16) uint8_t smem[ROWS * K3_KS * 2];  // activation slice, then the wave partials
+    constexpr int PK = K3_KS / PASS;                                     // k of a pass
+    constexpr int ACT = ROWS * PK * 2, PART = 4 * MB * 4 * 256 * 4;  // activations of a pass, wave partials
+    __shared__ __align__(16) uint8_t smem[ACT > PART ? ACT : PART];
+    __shared__ int big_l[PASS][4];
+    auto swz = [](int r, int c) { return r * (PK * 2) + ((c ^ (r & 7)) << 4); };
     const int t = threadIdx.x, lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const int n0 = blockIdx.x * K3_NB;
     const int slice = blockIdx.y;
     const int ks = slice * K3_KS;
-    const int klen = min(K3_KS, K - ks);  // multiple of 128
-    const int steps = klen >> 5;
+    const int groups = min(K3_KS, K - ks) >> 7;  // of the slice
     const int c4 = lane & 15, kq = lane >> 4;
     // Column quad of this lane; quads at or beyond N load the last valid quad (results dropped).
     const int ncol = min(n0 + 4 * c4, N - 4);
 
     // ---- loads, in the order their data is needed (vector loads return in
-    // issue order, so a wait for one load is a wait for every earlier one):
-    // the activation slice, then the slice's zero points and scales, then the
-    // weights, which keep streaming in while the first k-steps run.
-    // Activation slice (row r: 128 chunks of 16 bytes).  Rows at or beyond M
-    // are not loaded: their LDS rows are zero and their results dropped.
-    constexpr int CH = ROWS * (K3_KS / 8);  // 16-byte chunks
-    constexpr int PER = CH / 256;
-    // A buffer resource over the M rows: a load at or past its end returns
-    // zeros without a memory access, so the loads stay unconditional (a load
-    // under a branch makes the compiler wait for it at the join).
+    // issue order, so a wait for one load is a wait for every earlier one): the
+    // first pass's activations, the zero points and scales, the weights, which
+    // keep streaming in while the first pass runs.
+    // Activations of a pass (row r: PK / 8 octets of 16 bytes).  A buffer resource
+    // over the M rows: rows past it read as zeros, and octets past K (a
+    // partial slice) are never used.
+    constexpr int PER = ROWS * (PK / 8) / 256;
     const __amdgpu_buffer_rsrc_t rx =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(x), (short)0, (int)((uint32_t)M * K * 2u), K3_RSRC_WORD3);
     v4u xv[PER];
+    auto load_x = [&](int h) {
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-        const int q = t + i * 256;
-        const int r = q >> 7, c = q & 127;
-        const int cc = min(c, (klen >> 3) - 1);
-        xv[i] = __builtin_bit_cast(v4u, __builtin_amdgcn_raw_buffer_load_b128(rx, (int)(((uint32_t)r * K + ks + cc * 8) * 2u), 0, 0));
-    }
-    // Wave w takes the 8 consecutive 32-k steps 8w .. 8w+7 (groups 2w, 2w+1
-    // of the slice).
+        for (int i = 0; i < PER; ++i) {
+            const int q = t + i * 256, r = q / (PK / 8), c = q % (PK / 8);
+            const int k = min(ks + h * PK + c * 8, K - 8);
+            xv[i] = __builtin_bit_cast(
+                v4u, __builtin_amdgcn_raw_buffer_load_b128(rx, (int)(((uint32_t)r * K + k) * 2u), 0, 0));
+        }
+    };
+    auto store_x = [&](int h) {
+        uint32_t top = 0;
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const int q = t + i * 256;
+            const v4u v = xv[i];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) top = max(top, max(v[e] & 0x7fffu, (v[e] >> 16) & 0x7fffu));
+            *reinterpret_cast<v4u*>(&smem[swz(q / (PK / 8), q % (PK / 8))]) = octet_order(v);
+        }
+        const uint64_t any = __ballot(top >= MC::HUGE_MAG);
+        if (lane == 0) big_l[h][wave] = any != 0;
+    };
+    load_x(0);
+    // Wave w takes groups w and 4 + w of the slice.
     uint32_t zw[2];
     uint2 sv[2];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-        const int g = (ks >> 7) + max(0, min(2 * wave + i, (klen >> 7) - 1));
+        const int g = (ks >> 7) + min(4 * i + wave, groups - 1);
         zw[i] = (uint32_t)qzeros[(int64_t)g * (N >> 3) + (ncol >> 3)];
         sv[i] = *reinterpret_cast<const uint2*>(scales + (int64_t)g * N + ncol);
     }
-    const int nst = min(8, steps - 8 * wave);  // steps of this wave (may be <= 0)
     v4u wq[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        const int st = max(0, min(8 * wave + i, steps - 1));
-        const int64_t row = (int64_t)((ks >> 3) + st * 4 + kq);
+        const int g = min(4 * (i >> 2) + wave, groups - 1);
+        const int64_t row = (int64_t)((ks >> 3) + g * 16 + (i & 3) * 4 + kq);
         wq[i] = *reinterpret_cast<const v4u*>(qweight + row * N + ncol);
     }
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-        const int q = t + i * 256;
-        *reinterpret_cast<v4u*>(&smem[k3_swz(q >> 7, q & 127)]) = xv[i];
-    }
+    store_x(0);
+    if constexpr (PASS == 2) load_x(1);
     __syncthreads();
 
-    v4f acc[MB][4];
+    v4f total[MB][4];
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[mb][j] = v4f{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < 4; ++j) total[mb][j] = v4f{0.f, 0.f, 0.f, 0.f};
     const int zsh = 16 * (c4 & 1);  // the quad's 4 zero-point nibbles within its qzeros word
-    // Per group and column: the scale (as the activation dtype rounds it)
-    // and the zero-point offset.
-    typename TR::deq dq[2][4];
+    uint32_t mask = MC::MASK, one = MC::ONE;
+    asm volatile("" : "+s"(mask), "+v"(one));
+    auto group = [&](auto H, auto LIT) {
+        int zp1[4];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+        for (int j = 0; j < 4; ++j) zp1[j] = (int)((zw[H] >> (zsh + 4 * j)) & 15u) + 1;
+        v4f acc[MB][4], sum[MB];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t h = ((j < 2 ? sv[i].x : sv[i].y) >> (16 * (j & 1))) & 0xffffu;
-            dq[i][j] = TR::prep((uint16_t)h, (int)((zw[i] >> (zsh + 4 * j)) & 15u) + 1);
-        }
-    auto kstep = [&](int i) {
-        const int st = 8 * wave + i;
-        typename TR::vec bop[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) bop[j] = TR::dequant8(wq[i][j], dq[i >> 2][j]);
-        const int c = st * 4 + kq;  // 16-byte chunk of the k-octet in the slice row
-#pragma unroll
-        for (int mb = 0; mb < MB; ++mb) {
-            const v4u av = *reinterpret_cast<const v4u*>(&smem[k3_swz(mb * 16 + c4, c)]);
-            const typename TR::vec aop = __builtin_bit_cast(typename TR::vec, av);
+        for (int i = 0; i < 4; ++i) {
+            vec b[4];
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                if constexpr (XF16)
-                    acc[mb][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(aop, bop[j], acc[mb][j], 0, 0, 0);
+                if constexpr (LIT)
+                    b[j] = unbiased<XF16>(wq[4 * H + i][j], zp1[j]);
                 else
-                    acc[mb][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(aop, bop[j], acc[mb][j], 0, 0, 0);
+                    b[j] = MC::biased(wq[4 * H + i][j], mask, one);
+            }
+            const v4u ones = {one, one, one, one};
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb) {
+                const vec a = __builtin_bit_cast(
+                    vec, *reinterpret_cast<const v4u*>(&smem[swz(mb * 16 + c4, ((PASS == 1 ? 4 * H : 0) + wave) * 16 + i * 4 + kq)]));
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[mb][j] = MC::mma16(a, b[j], i ? acc[mb][j] : v4f{});
+                if constexpr (!LIT) sum[mb] = MC::mma16(a, __builtin_bit_cast(vec, ones), i ? sum[mb] : v4f{});
             }
         }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const uint32_t h = ((j < 2 ? sv[H].x : sv[H].y) >> (16 * (j & 1))) & 0xffffu;
+            const float s = MC::scale_of(h) * (LIT ? 1.0f : 16.0f), c = (float)(16 + zp1[j]) * 0.0625f;
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    float d = acc[mb][j][e];
+                    if constexpr (!LIT) d = __builtin_fmaf(-c, sum[mb][e], d);
+                    total[mb][j][e] = __builtin_fmaf(s, d, total[mb][j][e]);
+                }
+        }
     };
-    // A full slice gives every wave all 8 steps: that loop has no branch, so
-    // the weight loads stay where they were issued and each step waits only
-    // for its own (a load used only under a branch is moved into it and
-    // waited for there in full).
-    if (nst == 8) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) kstep(i);
-    } else {
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-            if (i < nst) kstep(i);  // uniform over the wave
+    auto half = [&](auto H) {
+        if (4 * H + wave < groups) {  // uniform over the wave
+            const int* big = big_l[PASS == 2 ? (int)H : 0];
+            if (big[0] | big[1] | big[2] | big[3])
+                group(H, std::true_type{});
+            else
+                group(H, std::false_type{});
+        }
+    };
+    half(std::integral_constant<int, 0>{});
+    if constexpr (PASS == 2) {
+        __syncthreads();  // the first half is read
+        store_x(1);
+        __syncthreads();
     }
-    __syncthreads();  // the activation slice is dead; its LDS takes the wave partials
+    half(std::integral_constant<int, 1>{});
+    __syncthreads();  // the activations are dead; their LDS takes the wave partials
+    v4f (&acc)[MB][4] = total;
     float* part = reinterpret_cast<float*>(smem);  // [wave][mb][j][256]
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
@@ -424,12 +466,6 @@ __device__ __forceinline__ typename BiasCode<F16>::vec biased8(uint32_t w) {
     const uint32_t m = 0x000F000Fu, hi = BiasCode<F16>::HI;
     const v4u r = {(w & m) | hi, ((w >> 4) & m) | hi, ((w >> 8) & m) | hi, ((w >> 12) & m) | hi};
     return __builtin_bit_cast(typename BiasCode<F16>::vec, r);
-}
-
-// An activation octet x0..x7 (16-bit pairs) reordered to x0 x4 x1 x5 x2 x6 x3 x7.
-__device__ __forceinline__ v4u octet_order(v4u v) {
-    return v4u{__builtin_amdgcn_perm(v[2], v[0], 0x05040100u), __builtin_amdgcn_perm(v[2], v[0], 0x07060302u),
-               __builtin_amdgcn_perm(v[3], v[1], 0x05040100u), __builtin_amdgcn_perm(v[3], v[1], 0x07060302u)};
 }
 
 // 16 bytes per lane from a buffer straight into LDS: lane l's bytes land at
@@ -707,8 +743,21 @@ template <int MB, bool XF, bool OF>
 hipError_t launch_dec(const void* x, const int32_t* qw, const int32_t* qz, const void* sc, void* out, float* ws,
                       int M, int N, int K, hipStream_t st) {
     const int S = (K + K3_KS - 1) / K3_KS;
-    hipLaunchKernelGGL((k3_dec<MB, XF>), dim3((unsigned)((N + K3_NB - 1) / K3_NB), (unsigned)S), dim3(256), 0, st,
-                       static_cast<const uint16_t*>(x), qw, qz, static_cast<const uint16_t*>(sc), ws, M, N, K);
+    const dim3 grid((unsigned)((N + K3_NB - 1) / K3_NB), (unsigned)S);
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, static_cast<const uint16_t*>(x), qw, qz,
+                           static_cast<const uint16_t*>(sc), ws, M, N, K);
+    };
+    // One pass over the slice where every workgroup has a CU to itself anyway
+    // (64 rows [4096 x 4096]: 12.3 us against 12.6 in two; with three workgroups
+    // per CU, [4096 x 12288], two passes take 24.6 against 28.1).  Same bits:
+    // the order of the groups does not change.
+    bool whole = false;
+    if constexpr (MB > 2) whole = (int64_t)grid.x * S <= device_cu_count();
+    if (whole)
+        go(k3_dec<MB, XF, (MB > 2 ? 1 : 2)>);
+    else
+        go(k3_dec<MB, XF, 2>);
     const int64_t MN = (int64_t)M * N;  // N % 8 == 0, so MN % 4 == 0
     hipLaunchKernelGGL((k3_reduce<OF>), dim3((unsigned)((MN / 4 + 255) / 256)), dim3(256), 0, st, ws, out, MN, S);
     return hipGetLastError();
