@@ -321,7 +321,8 @@ int nv4_w4a16_one_launch(int64_t M, int64_t N, int64_t K);
  * split into 1024-deep slices, each written as an fp32 partial [S, M, N]
  * (S = ceil(K/1024)) and then added in slice order and rounded once, so the
  * result is deterministic (not bit-identical to nv4_w4a16_gemm, whose
- * summation order differs).  workspace_bytes >= S*M*N*4, 16-byte aligned;
+ * summation order differs; the dequantized weights are not rounded to 16 bits).
+ * workspace_bytes >= S*M*N*4, 16-byte aligned;
  * qweight and x 16-byte aligned, scales and out 8-byte aligned.
  */
 int nv4_w4a16_gemm_ws(const void* x, int x_dtype, const int32_t* qweight, const int32_t* qzeros,
