@@ -33,7 +33,7 @@
  *   nv4_w4a4_weights_to_f6, nv4_w4a4_weights_f6_bytes <- no counterpart in the
  *                          reference: the weight half of that conversion, done
  *                          once per layer and kept beside the INT4 weights
- *   nv4_w4a16_gemm, nv4_w4a16_gemm_ws, nv4_w4a16_gemm_mid, nv4_w4a16_dequant <- nanovllm/layers/linear_w4a16.py:11
+ *   nv4_w4a16_gemm, nv4_w4a16_gemm_ws, nv4_w4a16_gemm_mid, nv4_w4a16_mid_form, nv4_w4a16_dequant <- nanovllm/layers/linear_w4a16.py:11
  *                          tl_dequant_matmul_w4a16 (called from W4A16Linear.forward
  *                          :128-148; the reference splits K 8 ways with bf16 atomics,
  *                          the _ws form splits K into 1024-deep fp32 partials, and
@@ -333,11 +333,13 @@ int nv4_w4a16_gemm_ws(const void* x, int x_dtype, const int32_t* qweight, const 
  * nv4_w4a16_gemm for prefill-sized M (any M >= 1 is taken), on the 32 x 32
  * matrix cores with a caller workspace (nv4_w4a16_gemm_mid_workspace bytes, or
  * -1 for sizes it does not take; 16-byte aligned): x is reordered once into
- * the workspace with its group sums, and where the tiles do not fill the
- * device K is split into fp32 partials added in slice order.  The dequantized
- * weights are not rounded to 16 bits; deterministic.  x 16-byte, qweight and
- * out 8-byte, scales 4-byte aligned.
+ * the workspace, and where the tiles do not fill the device K is split into
+ * fp32 partials added in slice order (how many depends on M and N).  The
+ * dequantized weights are not rounded to 16 bits; deterministic.  x 16-byte,
+ * qweight and out 8-byte, scales 4-byte aligned.  nv4_w4a16_mid_form: whether
+ * it is the fastest form for M rows of this type on the current device (1).
  */
+int nv4_w4a16_mid_form(int64_t M, int64_t N, int x_dtype);
 int64_t nv4_w4a16_gemm_mid_workspace(int64_t M, int64_t N, int64_t K);
 int nv4_w4a16_gemm_mid(const void* x, int x_dtype, const int32_t* qweight, const int32_t* qzeros,
                        const void* scales, void* out, int out_dtype, void* workspace, int64_t workspace_bytes,

@@ -1,31 +1,68 @@
-// GPTQ codes as 16-bit matrix operands, for the W4A16 GEMMs that apply scale
-// and zero point per quantisation group instead of per weight.
+// GPTQ codes as 16-bit matrix operands, for the W4A16 GEMMs that apply the scale
+// per quantisation group instead of per weight.
 //
-// A code q becomes (16 + q) / 16, exact in both types, by a shift and an
-// and-or per two codes of a word: a group (128 k) of an output is then
-//   sum x (q - z - 1) s = 16 s (S - (16 + z + 1) / 16 X),
-// S the product with the codes and X the row's sum of x over the group.  Rows
-// of HUGE_MAG and more (2^100; in fp16 infinities and NaN) would turn the bias
-// into NaN or into lost digits: they take the unbiased integer codes.
+// A code q becomes (q - z - 1) / 16, exact in both types, so a group (128 k) of
+// an output is 16 s S, S the product with these operands: one fma.  The zero
+// point comes off each code and not off the group's sum: codes biased to (16 + q)
+// / 16 and a correction by the row's sum of x cost fewer operations in bf16 (8
+// per word of eight codes against 17; fp16 8 against 9), but an element far
+// larger than its group then drowns the others' digits even where its weight
+// is 0 (bf16, one 2^30 among 1: 0.3 of the result in the columns whose code there
+// is the zero point; fp16, one 6e4 among 0.01: 3e-2).
 #pragma once
 
 #include "nv4_common.h"
 
 namespace nv4 {
 
+// An activation octet x0..x7 (16-bit pairs) reordered to x0 x4 x1 x5 x2 x6 x3 x7,
+// the order in which a word's codes come out.
+__device__ __forceinline__ v4u octet_order(v4u v) {
+    return v4u{__builtin_amdgcn_perm(v[2], v[0], 0x05040100u), __builtin_amdgcn_perm(v[2], v[0], 0x07060302u),
+               __builtin_amdgcn_perm(v[3], v[1], 0x05040100u), __builtin_amdgcn_perm(v[3], v[1], 0x07060302u)};
+}
+
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+
+// The eight codes of a word as fp16 pairs (0, 4) (1, 5) (2, 6) (3, 7): 1024 + q
+// where a code lies in the lowest four bits of a half, 1024 + 16 q in the next
+// four.  low: 0x000F000F, base: 0x64006400, one of them in a scalar and one in a
+// vector register (and-or takes no literals).
+__device__ __forceinline__ void code_pairs(uint32_t w, uint32_t low, uint32_t base, uint32_t (&h)[4]) {
+    const uint32_t v = w >> 8;
+    h[0] = (w & low) | base, h[1] = (w & (low << 4)) | base;
+    h[2] = (v & low) | base, h[3] = (v & (low << 4)) | base;
+}
+constexpr uint32_t K3_LOW = 0x000F000Fu, K3_BASE = 0x64006400u;
+
 template <bool F16>
-struct MidCode;
+struct K3Code;
 template <>
-struct MidCode<false> {
+struct K3Code<false> {
     typedef v8bf vec;
-    static constexpr uint32_t ONE = 0x3F803F80u, MASK = 0x00780078u, HUGE_MAG = 0x7180u;  // 2^100
+    static constexpr int OPS = 18;  // vector operations per word
+    struct zero {                   // of a column and group: for 1024 + q and for 1024 + 16 q
+        float a, b;
+    };
     __device__ static inline float scale_of(uint32_t s) {
         return bf16_to_f32(f32_to_bf16_rne((float)__builtin_bit_cast(_Float16, (uint16_t)s)));
     }
-    __device__ static inline float to_f32(uint32_t h) { return bf16_to_f32(h); }
-    // m, one: MASK and ONE in registers (one scalar, one vector: and-or takes no literals)
-    __device__ static inline vec biased(uint32_t w, uint32_t m, uint32_t one) {
-        const v4u r = {((w << 3) & m) | one, ((w >> 1) & m) | one, ((w >> 5) & m) | one, ((w >> 9) & m) | one};
+    __device__ static inline zero zero_of(int zp1) {
+        const float z = -0.0625f * (float)zp1;
+        return {z - 64.0f, z - 4.0f};
+    }
+    // fp16 to fp32 where the scaling, the subtraction and the widening are one
+    // operation; the bf16 values are the upper halves.
+    __device__ static inline uint32_t two(uint32_t h, float f, float z) {
+        const v2h v = __builtin_bit_cast(v2h, h);
+        const float lo = __builtin_fmaf((float)v[0], f, z), hi = __builtin_fmaf((float)v[1], f, z);
+        return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
+    }
+    __device__ static inline vec codes(uint32_t w, const zero& z, uint32_t low, uint32_t base) {
+        uint32_t h[4];
+        code_pairs(w, low, base, h);
+        const v4u r = {two(h[0], 0x1p-4f, z.a), two(h[1], 0x1p-8f, z.b), two(h[2], 0x1p-4f, z.a),
+                       two(h[3], 0x1p-8f, z.b)};
         return __builtin_bit_cast(vec, r);
     }
     __device__ static inline uint32_t of_f32(float f) { return f32_to_bf16_rne(f); }
@@ -37,13 +74,28 @@ struct MidCode<false> {
     }
 };
 template <>
-struct MidCode<true> {
+struct K3Code<true> {
     typedef v8h vec;
-    static constexpr uint32_t ONE = 0x3C003C00u, MASK = 0x03C003C0u, HUGE_MAG = 0x7C00u;  // infinities and NaN
+    static constexpr int OPS = 10;
+    struct zero {
+        v2h a, b;
+    };
     __device__ static inline float scale_of(uint32_t s) { return (float)__builtin_bit_cast(_Float16, (uint16_t)s); }
-    __device__ static inline float to_f32(uint32_t h) { return (float)__builtin_bit_cast(_Float16, (uint16_t)h); }
-    __device__ static inline vec biased(uint32_t w, uint32_t m, uint32_t one) {
-        const v4u r = {((w << 6) & m) | one, ((w << 2) & m) | one, ((w >> 2) & m) | one, ((w >> 6) & m) | one};
+    __device__ static inline zero zero_of(int zp1) {
+        const float z = -0.0625f * (float)zp1;
+        const _Float16 a = (_Float16)(z - 64.0f), b = (_Float16)(z - 4.0f);  // at most 11 bits: exact
+        return {v2h{a, a}, v2h{b, b}};
+    }
+    __device__ static inline vec codes(uint32_t w, const zero& z, uint32_t low, uint32_t base) {
+        uint32_t h[4];
+        code_pairs(w, low, base, h);
+        v4u r;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const _Float16 f = i & 1 ? (_Float16)0x1p-8f : (_Float16)0x1p-4f;
+            r[i] = __builtin_bit_cast(
+                uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(v2h, h[i]), v2h{f, f}, i & 1 ? z.b : z.a));
+        }
         return __builtin_bit_cast(vec, r);
     }
     __device__ static inline uint32_t of_f32(float f) {
@@ -56,15 +108,5 @@ struct MidCode<true> {
         return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
     }
 };
-
-// Integer codes q - zp1 of a word, in the order of biased().
-template <bool F16>
-__device__ __forceinline__ typename MidCode<F16>::vec unbiased(uint32_t w, int zp1) {
-    uint32_t h[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) h[e] = MidCode<F16>::of_f32((float)((int)((w >> (4 * e)) & 15u) - zp1));
-    const v4u r = {h[0] | (h[4] << 16), h[1] | (h[5] << 16), h[2] | (h[6] << 16), h[3] | (h[7] << 16)};
-    return __builtin_bit_cast(typename MidCode<F16>::vec, r);
-}
 
 }  // namespace nv4

@@ -25,6 +25,7 @@ struct Abi {
     decltype(&nv4_w4a4_linear) linear, linear_tiled, linear_rowtiled;
     decltype(&nv4_w4a16_gemm) w4a16;
     decltype(&nv4_w4a16_gemm_ws) w4a16_ws;
+    decltype(&nv4_w4a16_mid_form) w4a16_mid_form;
     decltype(&nv4_w4a16_gemm_mid) w4a16_mid;
     decltype(&nv4_w4a16_gemm_mid_workspace) w4a16_mid_bytes;
     decltype(&nv4_w4a16_one_launch) w4a16_one;
@@ -127,7 +128,7 @@ PyObject* dequant_matmul_w4a16(PyObject*, PyObject* const* args, Py_ssize_t n) {
             rc = abi.w4a16_ws(x.data_ptr(), code, qwp, qzp, sc.data_ptr(), out.data_ptr(), code,
                               static_cast<float*>(ws.data_ptr()), ws.numel() * 4, M, N, K, 128, st);
         } else {
-            const int64_t bytes = abi.w4a16_mid_bytes(M, N, K);
+            const int64_t bytes = abi.w4a16_mid_form(M, N, code) ? abi.w4a16_mid_bytes(M, N, K) : -1;
             if (bytes <= 0) Py_RETURN_NONE;
             const at::Tensor ws = at::empty({bytes}, x.options().dtype(at::kByte));
             rc = abi.w4a16_mid(x.data_ptr(), code, qwp, qzp, sc.data_ptr(), out.data_ptr(), code, ws.data_ptr(), bytes,

@@ -204,44 +204,37 @@ k3_w4a16(const uint16_t* __restrict__ x, const int32_t* __restrict__ qweight,
 //    by row, in the order in which a word's codes come out), so that two
 //    workgroups share a CU and one computes while the other loads;
 //  * dequantization per group (k3_codes.h): wave w takes group w of each half,
-//    four steps of biased codes and an all-ones MFMA for the rows' sums, then
-//    two fmas per output; rows with huge magnitudes run on unbiased codes;
+//    four steps of exact codes less their zero points, the next step's codes
+//    made between a step's MFMAs, then one fma per output;
 //  * the four waves' fp32 tiles are added in wave order in LDS, and the slice's
 //    [M, N] fp32 partial goes to the workspace; a second kernel adds the slices
 //    in order and rounds once (no atomics, same bits on every run, and for each
 //    column the same whatever N is).
 // Bound: 33..64 rows by the dequantizing VALU beside the MFMAs (a word's eight
-// codes cost 8 operations; scaling and rounding each weight cost about 24),
-// below that by the weight stream.  us with both launches, cold weights,
-// against a whole-slice form that scaled each weight: [6144 x 4096] 45 rows
-// 16.8 -> 14.3, 64 rows 19.8 -> 17.9; [24576 x 4096] 17 rows 24.2 -> 21.6,
-// 45 rows 41.9 -> 31.5, 64 rows 49.4 -> 39.7; [4096 x 12288] 45 rows 24.5 ->
-// 20.1, 64 rows 28.1 -> 24.6; [4096 x 4096] unchanged.  The distance to the
-// 64-bit product falls too, bf16 2.3e-3 -> 1.7e-3 (the rounding of the result).
+// codes cost 17 operations in bf16 and 9 in fp16; scaling and rounding each
+// weight cost about 24), below that by the weight stream.  us per call with both
+// launches, cold weights, bf16 / fp16, against a whole-slice form that scaled each
+// weight: [6144 x 4096] 45 rows 18.6 -> 13.8 / 13.1, 64 rows 19.7 -> 16.0 / 15.2;
+// [24576 x 4096] 17 rows 23.9 -> 20.7 / 19.1, 45 rows 41.8 -> 28.8 / 27.6, 64
+// rows 50.0 -> 36.1 / 34.9; [4096 x 12288] 17 rows 19.7 -> 16.2 / 14.9, 45 rows
+// 24.5 -> 19.6 / 18.9, 64 rows 28.5 -> 22.9 / 21.8.  A step's codes made in front
+// of its own MFMAs: [24576 x 4096] 45 rows 32.8 / 30.5, 64 rows 39.8 / 38.3.
 // ----------------------------------------------------------------------------
-// An activation octet x0..x7 (16-bit pairs) reordered to x0 x4 x1 x5 x2 x6 x3 x7.
-__device__ __forceinline__ v4u octet_order(v4u v) {
-    return v4u{__builtin_amdgcn_perm(v[2], v[0], 0x05040100u), __builtin_amdgcn_perm(v[2], v[0], 0x07060302u),
-               __builtin_amdgcn_perm(v[3], v[1], 0x05040100u), __builtin_amdgcn_perm(v[3], v[1], 0x07060302u)};
-}
-
 constexpr int K3_KS = 1024;  // k per slice
 constexpr int K3_RSRC_WORD3 = 0x00020000;  // buffer resource word 3 (CDNA): 32-bit data format
 constexpr int K3_NB = 64;    // columns per workgroup
-
 
 // PASS: passes over the activations in LDS, 1 (the whole slice) or 2 (halves).
 template <int MB, bool XF16, int PASS>
 __global__ void __launch_bounds__(256, PASS)
 k3_dec(const uint16_t* __restrict__ x, const int32_t* __restrict__ qweight, const int32_t* __restrict__ qzeros,
        const uint16_t* __restrict__ scales, float* __restrict__ ws, int M, int N, int K) {
-    using MC = MidCode<XF16>;
+    using MC = K3Code<XF16>;
     using vec = typename MC::vec;
     constexpr int ROWS = MB * 16;
     constexpr int PK = K3_KS / PASS;                                     // k of a pass
     constexpr int ACT = ROWS * PK * 2, PART = 4 * MB * 4 * 256 * 4;  // activations of a pass, wave partials
     __shared__ __align__(16) uint8_t smem[ACT > PART ? ACT : PART];
-    __shared__ int big_l[PASS][4];
     auto swz = [](int r, int c) { return r * (PK * 2) + ((c ^ (r & 7)) << 4); };
     const int t = threadIdx.x, lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -273,18 +266,12 @@ k3_dec(const uint16_t* __restrict__ x, const int32_t* __restrict__ qweight, cons
                 v4u, __builtin_amdgcn_raw_buffer_load_b128(rx, (int)(((uint32_t)r * K + k) * 2u), 0, 0));
         }
     };
-    auto store_x = [&](int h) {
-        uint32_t top = 0;
+    auto store_x = [&]() {
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
             const int q = t + i * 256;
-            const v4u v = xv[i];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) top = max(top, max(v[e] & 0x7fffu, (v[e] >> 16) & 0x7fffu));
-            *reinterpret_cast<v4u*>(&smem[swz(q / (PK / 8), q % (PK / 8))]) = octet_order(v);
+            *reinterpret_cast<v4u*>(&smem[swz(q / (PK / 8), q % (PK / 8))]) = octet_order(xv[i]);
         }
-        const uint64_t any = __ballot(top >= MC::HUGE_MAG);
-        if (lane == 0) big_l[h][wave] = any != 0;
     };
     load_x(0);
     // Wave w takes groups w and 4 + w of the slice.
@@ -303,7 +290,7 @@ k3_dec(const uint16_t* __restrict__ x, const int32_t* __restrict__ qweight, cons
         const int64_t row = (int64_t)((ks >> 3) + g * 16 + (i & 3) * 4 + kq);
         wq[i] = *reinterpret_cast<const v4u*>(qweight + row * N + ncol);
     }
-    store_x(0);
+    store_x();
     if constexpr (PASS == 2) load_x(1);
     __syncthreads();
 
@@ -313,60 +300,56 @@ k3_dec(const uint16_t* __restrict__ x, const int32_t* __restrict__ qweight, cons
 #pragma unroll
         for (int j = 0; j < 4; ++j) total[mb][j] = v4f{0.f, 0.f, 0.f, 0.f};
     const int zsh = 16 * (c4 & 1);  // the quad's 4 zero-point nibbles within its qzeros word
-    uint32_t mask = MC::MASK, one = MC::ONE;
-    asm volatile("" : "+s"(mask), "+v"(one));
-    auto group = [&](auto H, auto LIT) {
-        int zp1[4];
+    uint32_t low = K3_LOW, base = K3_BASE;
+    asm volatile("" : "+s"(low), "+v"(base));
+    auto half = [&](auto H) {
+        if (4 * H + wave >= groups) return;  // uniform over the wave
+        typename MC::zero z[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) zp1[j] = (int)((zw[H] >> (zsh + 4 * j)) & 15u) + 1;
-        v4f acc[MB][4], sum[MB];
+        for (int j = 0; j < 4; ++j) z[j] = MC::zero_of((int)((zw[H] >> (zsh + 4 * j)) & 15u) + 1);
+        v4f acc[MB][4];
+        vec a[2][MB], b[2][4];
+        auto operands = [&](auto i) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            vec b[4];
+            for (int mb = 0; mb < MB; ++mb)
+                a[i & 1][mb] = __builtin_bit_cast(
+                    vec, *reinterpret_cast<const v4u*>(
+                             &smem[swz(mb * 16 + c4, ((PASS == 1 ? 4 * H : 0) + wave) * 16 + i * 4 + kq)]));
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                if constexpr (LIT)
-                    b[j] = unbiased<XF16>(wq[4 * H + i][j], zp1[j]);
-                else
-                    b[j] = MC::biased(wq[4 * H + i][j], mask, one);
-            }
-            const v4u ones = {one, one, one, one};
-#pragma unroll
-            for (int mb = 0; mb < MB; ++mb) {
-                const vec a = __builtin_bit_cast(
-                    vec, *reinterpret_cast<const v4u*>(&smem[swz(mb * 16 + c4, ((PASS == 1 ? 4 * H : 0) + wave) * 16 + i * 4 + kq)]));
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[mb][j] = MC::mma16(a, b[j], i ? acc[mb][j] : v4f{});
-                if constexpr (!LIT) sum[mb] = MC::mma16(a, __builtin_bit_cast(vec, ones), i ? sum[mb] : v4f{});
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t h = ((j < 2 ? sv[H].x : sv[H].y) >> (16 * (j & 1))) & 0xffffu;
-            const float s = MC::scale_of(h) * (LIT ? 1.0f : 16.0f), c = (float)(16 + zp1[j]) * 0.0625f;
+            for (int j = 0; j < 4; ++j) b[i & 1][j] = MC::codes(wq[4 * H + i][j], z[j], low, base);
+        };
+        operands(std::integral_constant<int, 0>{});
+        // Codes and activations of the next step between this one's MFMAs.
+        static_for<0, 4>([&](auto i) {
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (i < 3) operands(std::integral_constant<int, i + 1>{});
 #pragma unroll
             for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    float d = acc[mb][j][e];
-                    if constexpr (!LIT) d = __builtin_fmaf(-c, sum[mb][e], d);
-                    total[mb][j][e] = __builtin_fmaf(s, d, total[mb][j][e]);
+                for (int j = 0; j < 4; ++j)
+                    acc[mb][j] = MC::mma16(a[i & 1][mb], b[i & 1][j], i == 0 ? v4f{} : acc[mb][j]);
+            if constexpr (i < 3) {
+#pragma unroll
+                for (int n = 0; n < 4 * MB; ++n) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                         // MFMA
+                    __builtin_amdgcn_sched_group_barrier(0x002, (MC::OPS + MB - 1) / MB, 0);  // VALU
                 }
-        }
-    };
-    auto half = [&](auto H) {
-        if (4 * H + wave < groups) {  // uniform over the wave
-            const int* big = big_l[PASS == 2 ? (int)H : 0];
-            if (big[0] | big[1] | big[2] | big[3])
-                group(H, std::true_type{});
-            else
-                group(H, std::false_type{});
+            }
+        });
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const uint32_t h = ((j < 2 ? sv[H].x : sv[H].y) >> (16 * (j & 1))) & 0xffffu;
+            const float s = MC::scale_of(h) * 16.0f;
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) total[mb][j][e] = __builtin_fmaf(s, acc[mb][j][e], total[mb][j][e]);
         }
     };
     half(std::integral_constant<int, 0>{});
     if constexpr (PASS == 2) {
         __syncthreads();  // the first half is read
-        store_x(1);
+        store_x();
         __syncthreads();
     }
     half(std::integral_constant<int, 1>{});
@@ -749,9 +732,9 @@ hipError_t launch_dec(const void* x, const int32_t* qw, const int32_t* qz, const
                            static_cast<const uint16_t*>(sc), ws, M, N, K);
     };
     // One pass over the slice where every workgroup has a CU to itself anyway
-    // (64 rows [4096 x 4096]: 12.3 us against 12.6 in two; with three workgroups
-    // per CU, [4096 x 12288], two passes take 24.6 against 28.1).  Same bits:
-    // the order of the groups does not change.
+    // ([4096 x 4096], bf16: 33 rows 10.1 us against 10.5 in two, 64 rows equal;
+    // with three workgroups per CU, [4096 x 12288], 64 rows take 28.3 in one and
+    // 23.0 in two).  Same bits: the order of the groups does not change.
     bool whole = false;
     if constexpr (MB > 2) whole = (int64_t)grid.x * S <= device_cu_count();
     if (whole)

@@ -2,24 +2,18 @@
 // 32 x 32 matrix cores, without a dense weight.
 //
 // Reference: nanovllm/layers/linear_w4a16.py:11-59, w = (q - z - 1) * s with
-// the scale rounded to the activation type.  As in the decode kernel k3_rows,
-// the matrix cores see biased codes, here (16 + q) / 16 -- a shift and
-// an and-or per two codes of a word: bf16 0x3F80 | q << 3, fp16 0x3C00 | q << 6, exact -- and a
-// quantisation group (128 k) of an output is
-//   sum x (q - z - 1) s = 16 s (S - (16 + z + 1) / 16 X),
-// S the product with the codes and X the row's sum of x over the group: two
-// fp32 fmas per output and group.  The weights are not rounded to 16 bits, so
-// the result is nearer to the 64-bit product than the dense form's (2.4e-3
-// against 2.9e-3 relative in bf16, of which 1.7e-3 is the rounding of x s and
-// of the result).  Rows with magnitudes of 2^100 and more, infinities or NaN
-// would turn the bias into NaN or into lost digits: their row tile runs on
-// unbiased integer codes.
+// the scale rounded to the activation type.  The matrix cores see the exact
+// values (q - z - 1) / 16 (k3_codes.h), and a quantisation group (128 k) of an
+// output is 16 s S, S the product with them: one fp32 fma per output and group.
+// The weights are not rounded to 16 bits, so the result is the 64-bit product
+// but for fp32 sums and its own rounding (bf16 1.7e-3 relative against 2.9e-3
+// of the dense form; fp16 2.1e-4 against 2.9e-4).
 //
 // Two launches (three with K split):
 //  * k3_prep reorders x once into operand order: per 32 rows and group an
 //    8 KiB block [step of 16 k][lane][16 bytes], lane l = row l % 32, octet
 //    2 step + l / 32, the octet as x0 x4 x1 x5 x2 x6 x3 x7 (the order in which
-//    a word's codes come out); with it X and a flag for the rows above.
+//    a word's codes come out).
 //  * k3_mid: workgroup = 4 waves side by side in N, tile 32 RB rows x 128 CB
 //    columns.  x goes from memory into a three-stage LDS ring (contiguous KiB
 //    per load, no registers, conflict-free reads); each wave loads its own
@@ -30,14 +24,15 @@
 //
 // Deterministic: fixed order, no atomics.
 //
-// What bounds it: the vector ALUs and the matrix cores in turn -- per block of
-// 32 x 32 and group 8 MFMAs (15 ns each) against 32 fmas and 8 code operations
-// per word -- at 260 ns per block and SIMD with the chip full, 0.55 of the
-// bf16 matrix rate; below one tile per CU, its two or three launches.  Against
-// a dense 16-bit weight written and multiplied by the library (us per call, M =
-// 65 / 128 / 300 / 512): o 33 / 44 / 48 / 43 -> 20 / 25 / 31 / 38; qkv 36 / 45 /
-// 45 / 62 -> 23 / 27 / 36 / 47; down 72 / 106 / 119 / 107 -> 28 / 31 / 57 / 93;
-// gate_up 81 / 84 / 113 / 134 -> 44 / 46 / 78 / 114.
+// What bounds it: in bf16 the vector ALUs -- per block of 32 x 32 and group 84
+// operations (17 per word of codes, 16 fmas) beside 8 MFMAs --, in fp16 (52
+// operations) these and the matrix cores in turn; below one tile per CU, its two
+// or three launches.  Against a dense 16-bit weight written and multiplied by the
+// library (bf16, us per call, M = 65 / 128 / 300 / 512): o 35 / 46 / 49 / 44 ->
+// 19 / 23 / 30 / 39; qkv 37 / 46 / 46 / 62 -> 22 / 26 / 34 / 48; down 73 / 107 /
+// 120 / 109 -> 28 / 30 / 53 / 99; gate_up 83 / 87 / 108 / 129 -> 46 / 47 / 77 /
+// 116 (fp16 40 / 42 / 68 / 105).  Codes biased by 16 with the zero point taken off
+// the group's sum ran gate_up in 42 / 44 / 72 / 110 in either type.
 #include <algorithm>
 
 #include "k3_codes.h"
@@ -51,45 +46,29 @@ constexpr int K3M_BLOCK = 8192;  // 32 rows x 128 k of 16-bit activations
 
 // One workgroup per 32 rows and group: thread t moves octet t % 16 of rows
 // t / 16 and t / 16 + 16.  Rows past M become zeros.
-template <bool F16>
 __global__ void __launch_bounds__(256)
-k3_prep(const uint16_t* __restrict__ x, uint8_t* __restrict__ xp, float* __restrict__ xsum, int* __restrict__ flags,
-        int M, int K, int G) {
+k3_prep(const uint16_t* __restrict__ x, uint8_t* __restrict__ xp, int M, int K, int G) {
     const int rb = blockIdx.x / G, g = blockIdx.x - rb * G;
     const int t = threadIdx.x, o = t & 15;
-    uint32_t top = 0;
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         const int rr = (t >> 4) + 16 * i, row = rb * 32 + rr;
         v4u v = {0u, 0u, 0u, 0u};
         if (row < M) v = *reinterpret_cast<const v4u*>(x + (int64_t)row * K + g * 128 + o * 8);
-        float s = 0.0f;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            s += MidCode<F16>::to_f32(v[q] & 0xffffu) + MidCode<F16>::to_f32(v[q] >> 16);
-            top = max(top, max(v[q] & 0x7fffu, (v[q] >> 16) & 0x7fffu));
-        }
-#pragma unroll
-        for (int d = 1; d < 16; d <<= 1) s += __shfl_xor(s, d);
-        const v4u p = {__builtin_amdgcn_perm(v[2], v[0], 0x05040100u), __builtin_amdgcn_perm(v[2], v[0], 0x07060302u),
-                       __builtin_amdgcn_perm(v[3], v[1], 0x05040100u), __builtin_amdgcn_perm(v[3], v[1], 0x07060302u)};
-        *reinterpret_cast<v4u*>(xp + (int64_t)blockIdx.x * K3M_BLOCK + (o >> 1) * 1024 + ((o & 1) * 32 + rr) * 16) = p;
-        if (o == 0) xsum[(int64_t)blockIdx.x * 32 + rr] = s;
+        *reinterpret_cast<v4u*>(xp + (int64_t)blockIdx.x * K3M_BLOCK + (o >> 1) * 1024 + ((o & 1) * 32 + rr) * 16) =
+            octet_order(v);
     }
-    const int big = __syncthreads_or(top >= MidCode<F16>::HUGE_MAG);
-    if (t == 0) flags[blockIdx.x] = big;
 }
 
 template <int RB, int CB, bool XF16, bool OF16>
 __global__ void __launch_bounds__(256, 2)
 k3_mid(const uint8_t* __restrict__ xp, const int32_t* __restrict__ qweight, const int32_t* __restrict__ qzeros,
-       const uint16_t* __restrict__ scales, const float* __restrict__ xsum, const int* __restrict__ flags,
-       void* __restrict__ out, float* __restrict__ ws, int M, int N, int G, int tm, int tn, int T, int per_slice) {
-    using MC = MidCode<XF16>;
+       const uint16_t* __restrict__ scales, void* __restrict__ out, float* __restrict__ ws, int M, int N, int G, int tm, int tn, int T, int per_slice) {
+    using MC = K3Code<XF16>;
     using vec = typename MC::vec;
-    constexpr int STAGE = RB * K3M_BLOCK + 256;  // activations, then the row sums
-    constexpr int DMA = 2 * RB + 1;              // loads into LDS per wave and group
-    constexpr int WL = 10;                       // loads into registers per group: 8 of words, scales, zero points
+    constexpr int STAGE = RB * K3M_BLOCK;
+    constexpr int DMA = 2 * RB;  // loads into LDS per wave and group
+    constexpr int WL = 10;       // loads into registers per group: 8 of words, scales, zero points
     __shared__ __align__(16) uint8_t st[3 * STAGE];
 
     // Ids are dealt round-robin over the 8 XCDs; each gets a contiguous run of
@@ -105,13 +84,12 @@ k3_mid(const uint8_t* __restrict__ xp, const int32_t* __restrict__ qweight, cons
     const int n = nt * 128 * CB + wave * 32 * CB + CB * rc;  // the lane's first column
     const int nl = min(n, N - CB);                           // columns past N load the last ones, results dropped
 
-    // Activations and sums of the tile's row blocks (rows of blocks past M are
-    // zeros; a whole block past M lies past the resource).
+    // Activations of the tile's row blocks (rows of blocks past M are zeros; a
+    // whole block past M lies past the resource).
     const int nrb = min(RB, (M + 31) / 32 - mt * RB);
     const v4u rx = scalar_rsrc(xp + (int64_t)mt * RB * G * K3M_BLOCK, (uint32_t)(nrb * G * K3M_BLOCK));
-    const v4u rsum = scalar_rsrc(xsum + (int64_t)mt * RB * G * 32, (uint32_t)(nrb * G * 128));
     const uint32_t base = lds_address(st);
-    const uint32_t xoff = (uint32_t)(lane * 16), soff = (uint32_t)(half * G * 128 + rc * 4);
+    const uint32_t xoff = (uint32_t)(lane * 16);
     auto dma = [&](int g, int at) {
         const uint32_t from = g < gb ? (uint32_t)(g * K3M_BLOCK) : kOutOfRange;
 #pragma unroll
@@ -120,7 +98,6 @@ k3_mid(const uint8_t* __restrict__ xp, const int32_t* __restrict__ qweight, cons
             lds_load16(rx, xoff + (uint32_t)((piece >> 3) * G * K3M_BLOCK + (piece & 7) * 1024), from,
                        base + at + piece * 1024);
         }
-        lds_load4(rsum, soff, g < gb ? (uint32_t)(g * 128) : kOutOfRange, base + at + RB * K3M_BLOCK);
     };
     // Weights: word rows 16 g + 2 step + half, CB words from column n.
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
@@ -168,104 +145,73 @@ k3_mid(const uint8_t* __restrict__ xp, const int32_t* __restrict__ qweight, cons
         load_s(ga + X, X);
         __builtin_amdgcn_sched_barrier(0);
     });
-    // Rows that need unbiased codes, in any group of the slice (asked for after
-    // the first stages' loads).
-    bool big = false;
-#pragma unroll
-    for (int i = 0; i < RB; ++i)
-        for (int g = ga + lane; g < gb; g += 64) big |= i < nrb && flags[(int64_t)(mt * RB + i) * G + g] != 0;
-    big = __any(big);
-
-    uint32_t mask = MC::MASK, one = MC::ONE;
-    asm volatile("" : "+s"(mask), "+v"(one));
+    uint32_t low = K3_LOW, codes = K3_BASE;
+    asm volatile("" : "+s"(low), "+v"(codes));
     int cur = 0, next = STAGE, far = 2 * STAGE;  // stages of groups g, g + 1, g + 2
-    // A group past the slice (odd counts) has zero activations, sums and
-    // scales: it adds +0.
-    auto run = [&](auto LIT) {
-        for (int g0 = ga; g0 < gb; g0 += 2)
-            static_for<0, 2>([&](auto X) {
-                const int g = g0 + X;
-                // Younger than the stage of group g: the words of g, the stage
-                // and the words of g + 1.
-                lds_ring_barrier<WL + DMA + WL>();
-                dma(g + 2, far);
-                const uint32_t from = words_of(g + 2);
+    // A group past the slice (odd counts) has zero activations and scales: it adds +0.
+    for (int g0 = ga; g0 < gb; g0 += 2)
+        static_for<0, 2>([&](auto X) {
+            const int g = g0 + X;
+            // Younger than the stage of group g: the words of g, the stage
+            // and the words of g + 1.
+            lds_ring_barrier<WL + DMA + WL>();
+            dma(g + 2, far);
+            const uint32_t from = words_of(g + 2);
+            __builtin_amdgcn_sched_barrier(0);
+            float s16[CB];
+            typename MC::zero z[CB];
+#pragma unroll
+            for (int j = 0; j < CB; ++j) {
+                z[j] = MC::zero_of((int)((zr[X] >> (4 * ((nl + j) & 7))) & 15u) + 1);
+                s16[j] = MC::scale_of(j ? sr[X] >> 16 : sr[X] & 0xffffu) * 16.0f;
+            }
+            v16f acc[RB][CB];
+            vec a[2][RB];
+            auto read_a = [&](auto S) {
+#pragma unroll
+                for (int i = 0; i < RB; ++i)
+                    a[S & 1][i] = __builtin_bit_cast(
+                        vec, *reinterpret_cast<const v4u*>(st + cur + i * K3M_BLOCK + S * 1024 + lane * 16));
+            };
+            vec w[2][CB];
+            auto unpack = [&](auto S) {
+#pragma unroll
+                for (int j = 0; j < CB; ++j) w[S & 1][j] = MC::codes(wr[X][S][j], z[j], low, codes);
+                load_w(from, X, S);
+            };
+            read_a(std::integral_constant<int, 0>{});
+            unpack(std::integral_constant<int, 0>{});
+            // Codes and activations of the next step between this one's MFMAs.
+            static_for<0, 8>([&](auto S) {
                 __builtin_amdgcn_sched_barrier(0);
-                float s16[CB], c[CB];
-                int zp1[CB];
-#pragma unroll
-                for (int j = 0; j < CB; ++j) {
-                    zp1[j] = (int)((zr[X] >> (4 * ((nl + j) & 7))) & 15u) + 1;
-                    s16[j] = MC::scale_of(j ? sr[X] >> 16 : sr[X] & 0xffffu) * (LIT ? 1.0f : 16.0f);
-                    c[j] = LIT ? 0.0f : (float)(16 + zp1[j]) * 0.0625f;
+                if constexpr (S < 7) {
+                    read_a(std::integral_constant<int, S + 1>{});
+                    unpack(std::integral_constant<int, S + 1>{});
                 }
-                v16f acc[RB][CB];
-                vec a[2][RB];
-                auto read_a = [&](auto S) {
 #pragma unroll
-                    for (int i = 0; i < RB; ++i)
-                        a[S & 1][i] = __builtin_bit_cast(
-                            vec, *reinterpret_cast<const v4u*>(st + cur + i * K3M_BLOCK + S * 1024 + lane * 16));
-                };
-                vec w[2][CB];
-                auto unpack = [&](auto S) {
-#pragma unroll
-                    for (int j = 0; j < CB; ++j) {
-                        if constexpr (LIT)
-                            w[S & 1][j] = unbiased<XF16>(wr[X][S][j], zp1[j]);
-                        else
-                            w[S & 1][j] = MC::biased(wr[X][S][j], mask, one);
-                    }
-                    load_w(from, X, S);
-                };
-                read_a(std::integral_constant<int, 0>{});
-                unpack(std::integral_constant<int, 0>{});
-                // Codes and activations of the next step between this one's MFMAs.
-                static_for<0, 8>([&](auto S) {
-                    __builtin_amdgcn_sched_barrier(0);
-                    if constexpr (S < 7) {
-                        read_a(std::integral_constant<int, S + 1>{});
-                        unpack(std::integral_constant<int, S + 1>{});
-                    }
-#pragma unroll
-                    for (int i = 0; i < RB; ++i)
-#pragma unroll
-                        for (int j = 0; j < CB; ++j)
-                            acc[i][j] = MC::mma(a[S & 1][i], w[S & 1][j], S == 0 ? v16f{} : acc[i][j]);
-                    if constexpr (S < 7 && !LIT) {
-#pragma unroll
-                        for (int i = 0; i < RB * CB; ++i) {
-                            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);           // MFMA
-                            __builtin_amdgcn_sched_group_barrier(0x002, 8 / RB, 0);      // VALU
-                        }
-                    }
-                });
-                load_s(g + 2, X);
-#pragma unroll
-                for (int i = 0; i < RB; ++i) {
-                    v4f xs[4];
-#pragma unroll
-                    for (int q = 0; q < 4; ++q)
-                        xs[q] = *reinterpret_cast<const v4f*>(st + cur + RB * K3M_BLOCK + i * 128 +
-                                                              (8 * q + 4 * half) * 4);
+                for (int i = 0; i < RB; ++i)
 #pragma unroll
                     for (int j = 0; j < CB; ++j)
+                        acc[i][j] = MC::mma(a[S & 1][i], w[S & 1][j], S == 0 ? v16f{} : acc[i][j]);
+                if constexpr (S < 7) {
 #pragma unroll
-                        for (int v = 0; v < 16; ++v) {
-                            float d = acc[i][j][v];
-                            if constexpr (!LIT) d = __builtin_fmaf(-c[j], xs[v >> 2][v & 3], d);
-                            total[i][j][v] = __builtin_fmaf(s16[j], d, total[i][j][v]);
-                        }
+                    for (int i = 0; i < RB * CB; ++i) {
+                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);             // MFMA
+                        __builtin_amdgcn_sched_group_barrier(0x002, MC::OPS / RB, 0);  // VALU
+                    }
                 }
-                __builtin_amdgcn_sched_barrier(0);
-                const int free = cur;
-                cur = next, next = far, far = free;
             });
-    };
-    if (big)
-        run(std::true_type{});
-    else
-        run(std::false_type{});
+            load_s(g + 2, X);
+#pragma unroll
+            for (int i = 0; i < RB; ++i)
+#pragma unroll
+                for (int j = 0; j < CB; ++j)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) total[i][j][v] = __builtin_fmaf(s16[j], acc[i][j][v], total[i][j][v]);
+            __builtin_amdgcn_sched_barrier(0);
+            const int free = cur;
+            cur = next, next = far, far = free;
+        });
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no load may write LDS after the workgroup has gone
 
     if (n >= N) return;
@@ -283,9 +229,9 @@ k3_mid(const uint8_t* __restrict__ xp, const int32_t* __restrict__ qweight, cons
                     *p = total[i][0][v];
             } else {
                 uint16_t* p = static_cast<uint16_t*>(out) + (int64_t)m * N + n;
-                const uint32_t h0 = MidCode<OF16>::of_f32(total[i][0][v]);
+                const uint32_t h0 = K3Code<OF16>::of_f32(total[i][0][v]);
                 if constexpr (CB == 2)
-                    *reinterpret_cast<uint32_t*>(p) = h0 | (MidCode<OF16>::of_f32(total[i][CB - 1][v]) << 16);
+                    *reinterpret_cast<uint32_t*>(p) = h0 | (K3Code<OF16>::of_f32(total[i][CB - 1][v]) << 16);
                 else
                     *p = (uint16_t)h0;
             }
@@ -294,7 +240,7 @@ k3_mid(const uint8_t* __restrict__ xp, const int32_t* __restrict__ qweight, cons
 
 struct MidPlan {
     int rb, cb, slices, per_slice;
-    int64_t xp, sums, flags, partials;  // workspace bytes
+    int64_t xp, partials;  // workspace bytes
 };
 
 MidPlan plan_of(int64_t M, int64_t N, int64_t K) {
@@ -310,8 +256,6 @@ MidPlan plan_of(int64_t M, int64_t N, int64_t K) {
     p.per_slice = (int)((G + s - 1) / s);
     p.slices = (int)((G + p.per_slice - 1) / p.per_slice);
     p.xp = mb * G * K3M_BLOCK;
-    p.sums = mb * G * 128;
-    p.flags = (mb * G * 4 + 15) / 16 * 16;
     p.partials = p.slices > 1 ? (int64_t)p.slices * M * N * 4 : 0;
     return p;
 }
@@ -321,16 +265,14 @@ hipError_t launch_mid16(const MidPlan& p, const void* x, const int32_t* qw, cons
                         void* out, uint8_t* wsp, int M, int N, int K, hipStream_t st) {
     const int G = K / 128, mb = (M + 31) / 32;
     uint8_t* xp = wsp;
-    float* sums = reinterpret_cast<float*>(wsp + p.xp);
-    int* flags = reinterpret_cast<int*>(wsp + p.xp + p.sums);
-    float* part = p.slices > 1 ? reinterpret_cast<float*>(wsp + p.xp + p.sums + p.flags) : nullptr;
-    hipLaunchKernelGGL((k3_prep<XF>), dim3((unsigned)(mb * G)), dim3(256), 0, st, static_cast<const uint16_t*>(x), xp,
-                       sums, flags, M, K, G);
+    float* part = p.slices > 1 ? reinterpret_cast<float*>(wsp + p.xp) : nullptr;
+    hipLaunchKernelGGL(k3_prep, dim3((unsigned)(mb * G)), dim3(256), 0, st, static_cast<const uint16_t*>(x), xp, M, K,
+                       G);
     const int tm = (mb + p.rb - 1) / p.rb, tn = (N + 128 * p.cb - 1) / (128 * p.cb), T = tm * tn * p.slices;
     const auto* scp = static_cast<const uint16_t*>(sc);
     auto go = [&](auto RB, auto CB) {
-        hipLaunchKernelGGL((k3_mid<RB, CB, XF, OF>), dim3((unsigned)T), dim3(256), 0, st, xp, qw, qz, scp, sums, flags,
-                           out, part, M, N, G, tm, tn, T, p.per_slice);
+        hipLaunchKernelGGL((k3_mid<RB, CB, XF, OF>), dim3((unsigned)T), dim3(256), 0, st, xp, qw, qz, scp, out,
+                           part, M, N, G, tm, tn, T, p.per_slice);
     };
     using I1 = std::integral_constant<int, 1>;
     using I2 = std::integral_constant<int, 2>;
@@ -358,11 +300,24 @@ bool mid_shape(int64_t M, int64_t N, int64_t K) {
 }  // namespace
 }  // namespace nv4
 
+// Where this form beats the dense one.  fp16: every projection to 640 rows (us at
+// 640: o 42.3 / 46.9, qkv 45.4 / 54.9, down 108 / 117, gate_up 130 / 164).  bf16 has
+// more operations per code: all to 512 rows, and beyond not while the tiles are
+// more than one and less than 1.5 per CU, which take the time of two (o and down
+// at 544: 47.5 / 47.3 and 124 / 116; qkv and gate_up, 1.7 and 6.8 tiles per CU:
+// 48.3 / 50.7 and 142 / 155).
+extern "C" int nv4_w4a16_mid_form(int64_t M, int64_t N, int x_dtype) {
+    if (M <= 64 || M > 640 || N < 1) return 0;
+    if (x_dtype == NV4_FP16 || M <= 512) return 1;
+    const int64_t tiles = ((M + 63) / 64) * ((N + 127) / 128), cus = nv4::device_cu_count();
+    return tiles <= cus || 2 * tiles >= 3 * cus;
+}
+
 extern "C" int64_t nv4_w4a16_gemm_mid_workspace(int64_t M, int64_t N, int64_t K) {
     using namespace nv4;
     if (!mid_shape(M, N, K)) return -1;
     const MidPlan p = plan_of(M, N, K);
-    return p.xp + p.sums + p.flags + p.partials;
+    return p.xp + p.partials;
 }
 
 extern "C" int nv4_w4a16_gemm_mid(const void* x, int x_dtype, const int32_t* qweight, const int32_t* qzeros,
@@ -375,7 +330,7 @@ extern "C" int nv4_w4a16_gemm_mid(const void* x, int x_dtype, const int32_t* qwe
     if (group != 128) return NV4_E_GROUP;
     if (!mid_shape(M, N, K)) return NV4_E_SHAPE;
     const MidPlan p = plan_of(M, N, K);
-    if (workspace_bytes < p.xp + p.sums + p.flags + p.partials) return NV4_E_SHAPE;
+    if (workspace_bytes < p.xp + p.partials) return NV4_E_SHAPE;
     if (reinterpret_cast<uintptr_t>(x) % 16 || reinterpret_cast<uintptr_t>(qweight) % 8 ||
         reinterpret_cast<uintptr_t>(qzeros) % 4 || reinterpret_cast<uintptr_t>(scales) % 4 ||
         reinterpret_cast<uintptr_t>(out) % 8 || reinterpret_cast<uintptr_t>(workspace) % 16)

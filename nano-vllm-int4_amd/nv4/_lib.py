@@ -55,6 +55,7 @@ SIGNATURES = {
     "nv4_w4a16_gemm": ([_P, _I, _P, _P, _P, _P, _I, _I64, _I64, _I64, _I, _P], _I),
     "nv4_w4a16_one_launch": ([_I64, _I64, _I64], _I),
     "nv4_w4a16_gemm_ws": ([_P, _I, _P, _P, _P, _P, _I, _P, _I64, _I64, _I64, _I64, _I, _P], _I),
+    "nv4_w4a16_mid_form": ([_I64, _I64, _I], _I),
     "nv4_w4a16_gemm_mid_workspace": ([_I64, _I64, _I64], _I64),
     "nv4_w4a16_gemm_mid": ([_P, _I, _P, _P, _P, _P, _I, _P, _I64, _I64, _I64, _I64, _I, _P], _I),
     "nv4_w4a16_dequant": ([_P, _P, _P, _P, _I, _I64, _I64, _I, _P], _I),
@@ -89,7 +90,8 @@ _lock = threading.Lock()
 
 # What nv4._ops calls, in the order of its entry-point table.
 _OPS_ENTRIES = ("nv4_w4a4_linear", "nv4_w4a4_linear_tiled", "nv4_w4a4_linear_rowtiled", "nv4_w4a16_gemm",
-                "nv4_w4a16_gemm_ws", "nv4_w4a16_gemm_mid", "nv4_w4a16_gemm_mid_workspace", "nv4_w4a16_one_launch")
+                "nv4_w4a16_gemm_ws", "nv4_w4a16_mid_form", "nv4_w4a16_gemm_mid", "nv4_w4a16_gemm_mid_workspace",
+                "nv4_w4a16_one_launch")
 
 
 class NV4LibraryError(RuntimeError):

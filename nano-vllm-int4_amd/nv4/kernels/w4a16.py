@@ -21,8 +21,9 @@ workgroups are several per CU) take the split-K form
 fp32 partials into a workspace from torch's caching allocator, added in slice
 order by a second launch.  Both are deterministic and graph-capturable.
 
-65 to 640 rows (``mid_form``) run ``nv4_w4a16_gemm_mid``: the codes meet
-reordered activations on the 32 x 32 matrix cores, no dense weight in between.
+65 to 640 rows (``mid_form``) run ``nv4_w4a16_gemm_mid``: the codes less their
+zero points, exact in 16 bits, meet reordered activations on the 32 x 32 matrix
+cores, no dense weight in between.
 Beyond that the weight is
 dequantized once into a dense [K, N] tensor (``nv4_w4a16_dequant``, the same per-element
 rounding) and the product runs as a library GEMM (torch.mm on hipBLASLt,
@@ -76,14 +77,12 @@ def one_launch(M, N, K, device=None):
         return bool(_lib.load().nv4_w4a16_one_launch(M, N, K))
 
 
-def mid_form(M):
-    """Whether ``nv4_w4a16_gemm_mid`` serves M rows.  Against the dense weight
-    and the library's product it wins on every projection up to 640 rows (us
-    per call at 300 / 640: o 31, 48 against 48, 51; qkv 35, 57 / 45, 59; down 54,
-    121 / 119, 126; gate_up 77, 154 / 113, 175) and loses on qkv at 768 (71 / 63).
-    Up to 64 rows the results must not depend on N (fused projections equal the
-    separate ones bit for bit), which its K slices do."""
-    return SPLIT_MAX_M < M <= MID_MAX_M
+def mid_form(M, N=None, dtype=torch.float16):
+    """Whether ``nv4_w4a16_gemm_mid`` serves M rows of ``dtype`` (of N columns:
+    bf16 past 512 rows not on every grid; the library's rule)."""
+    if N is None:
+        return SPLIT_MAX_M < M <= MID_MAX_M
+    return bool(_lib.load().nv4_w4a16_mid_form(M, N, _DT[dtype]))
 
 
 def dequant_matmul_w4a16(x, qweight, qzeros, scales, group_size=128, out=None):
@@ -120,7 +119,7 @@ def dequant_matmul_w4a16(x, qweight, qzeros, scales, group_size=128, out=None):
                                     ctypes.c_void_p(qweight.data_ptr()), ctypes.c_void_p(qzeros.data_ptr()),
                                     ctypes.c_void_p(scales.data_ptr()), ctypes.c_void_p(out.data_ptr()),
                                     _DT[out.dtype], M, N, K, group_size, ctypes.c_void_p(stream))
-        elif (mid_form(M) and (nbytes := lib.nv4_w4a16_gemm_mid_workspace(M, N, K)) > 0
+        elif (mid_form(M, N, x.dtype) and (nbytes := lib.nv4_w4a16_gemm_mid_workspace(M, N, K)) > 0
               and not any(t.data_ptr() % 16 for t in (x, qweight, scales, out))):
             ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
             rc = lib.nv4_w4a16_gemm_mid(ctypes.c_void_p(x.data_ptr()), _DT[x.dtype],
