@@ -48,7 +48,11 @@ class W4A16Linear(nn.Module):
         # (after fuse_w4a16 the parameters are column views of the fused
         # tensors; a direct call then reads contiguous copies)
         p = self._parameters
-        weights = [p[name].contiguous() for name in ("qweight", "qzeros", "scales")]
+        try:  # by dict: nn.Module's attribute lookup costs more than the operator's checks
+            weights = p["qweight"], p["qzeros"], p["scales"]
+        except KeyError:  # a replica's copies, plain attributes, parametrizations
+            weights = self.qweight, self.qzeros, self.scales
+        weights = [w.contiguous() for w in weights]
         if x.ndim == 2 and x.shape[1] == self.in_features and x.is_contiguous():
             return dequant_matmul_w4a16(x, *weights, self.group_size)
         out = dequant_matmul_w4a16(x.reshape(-1, self.in_features).contiguous(), *weights, self.group_size)

@@ -132,16 +132,17 @@ class W4A4Linear(nn.Module):
             raise ValueError("W4A4Linear requires BF16 activations with the configured input width")
         # RHT + quantize + pack, then the grouped INT4 GEMM; packed codes and
         # scales come from the caching allocator, so the forward can be
-        # captured in a HIP graph.  (Buffers by dict: nn.Module's attribute
-        # lookup costs more than the checks.)
+        # captured in a HIP graph.
         b = self._buffers
+        try:  # by dict: nn.Module's attribute lookup costs more than the operator's checks
+            signs, packed, scale = b["signs"], b["packed_weight"], b["weight_scale"]
+        except KeyError:  # plain attributes, parametrizations
+            signs, packed, scale = self.signs, self.packed_weight, self.weight_scale
         if x.ndim == 2 and x.is_contiguous():
-            f6 = self._f6() if b["weight_f6"] is not None and x.shape[0] >= PREFILL_MIN_M else None
-            return w4a4_linear(x, b["signs"], b["packed_weight"], b["weight_scale"], weights_tiled=self.weights_tiled,
-                               weights_f6=f6)
+            f6 = self._f6() if x.shape[0] >= PREFILL_MIN_M else None
+            return w4a4_linear(x, signs, packed, scale, weights_tiled=self.weights_tiled, weights_f6=f6)
         flat = x.reshape(-1, self.in_features).contiguous()
-        out = w4a4_linear(flat, b["signs"], b["packed_weight"], b["weight_scale"], weights_tiled=self.weights_tiled,
-                          weights_f6=self._f6())
+        out = w4a4_linear(flat, signs, packed, scale, weights_tiled=self.weights_tiled, weights_f6=self._f6())
         return out.reshape(*x.shape[:-1], self.out_features)
 
     def uses_rowtiled(self, m: int) -> bool:
