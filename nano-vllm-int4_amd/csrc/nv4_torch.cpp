@@ -10,7 +10,9 @@
 // Whatever is not the plain case -- another type, shape, layout or device, a
 // tensor subclass, sizes another path serves, an error of any kind -- returns
 // None, and the caller goes on in its general path, which decides and raises
-// as it always has.  Nothing is kept between calls.
+// as it always has.  Nothing is kept between calls.  Allocation and launch run
+// without the interpreter lock, as torch's bindings and ctypes release it: either
+// may wait for the device, and other threads go on meanwhile.
 #include <ATen/ATen.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/DeviceGuard.h>
@@ -42,6 +44,10 @@ bool plain(PyObject* o) {
 bool is(const at::Tensor& t, at::ScalarType type, const at::Device& dev, int64_t dims) {
     return t.scalar_type() == type && t.device() == dev && t.dim() == dims && t.is_contiguous();
 }
+struct NoGil {
+    PyThreadState* const state = PyEval_SaveThread();
+    ~NoGil() { PyEval_RestoreThread(state); }
+};
 void* stream_of(const at::Device& dev) {
     return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(dev.index()).stream();
 }
@@ -59,8 +65,8 @@ PyObject* w4a4_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
         Py_RETURN_NONE;
     }
     try {
-        const at::Tensor &x = THPVariable_Unpack(args[0]), &signs = THPVariable_Unpack(args[1]),
-                         &w = THPVariable_Unpack(args[2]), &sw = THPVariable_Unpack(args[3]);
+        const at::Tensor x = THPVariable_Unpack(args[0]), signs = THPVariable_Unpack(args[1]),
+                         w = THPVariable_Unpack(args[2]), sw = THPVariable_Unpack(args[3]);
         if (!x.is_cuda()) Py_RETURN_NONE;
         const at::Device dev = x.device();
         if (!is(x, at::kBFloat16, dev, 2) || !is(signs, at::kChar, dev, 1) || !is(w, at::kChar, dev, 2) ||
@@ -70,17 +76,22 @@ PyObject* w4a4_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
         if ((K != 4096 && K != 12288) || M < 1 || M >= below || N < 8 || N % 8 || (tiled && N % 16) ||
             signs.size(0) != K || w.size(1) != K / 2 || sw.size(0) != N || sw.size(1) != K / 128)
             Py_RETURN_NONE;
-        const c10::DeviceGuard guard(dev);
-        const bool rowtiled = tiled && M <= rowtiled_max;
-        const int64_t rows = rowtiled ? (M + 15) / 16 * 16 : M;
-        at::Tensor out = at::empty({M, N}, x.options());
-        // Codes, then their scales (rows * K / 2 is a multiple of 2048).
-        const at::Tensor codes = at::empty({rows * (K / 2) + M * (K / 64)}, signs.options());
-        int8_t* packed = static_cast<int8_t*>(codes.data_ptr());
-        const auto fn = rowtiled ? abi.linear_rowtiled : tiled ? abi.linear_tiled : abi.linear;
-        const int rc = fn(x.data_ptr(), static_cast<const int8_t*>(signs.data_ptr()),
-                          static_cast<const int8_t*>(w.data_ptr()), sw.data_ptr(), out.data_ptr(), packed,
-                          packed + rows * (K / 2), M, N, K, stream_of(dev));
+        at::Tensor out;
+        int rc;
+        {
+            const NoGil released;
+            const c10::DeviceGuard guard(dev);
+            const bool rowtiled = tiled && M <= rowtiled_max;
+            const int64_t rows = rowtiled ? (M + 15) / 16 * 16 : M;
+            out = at::empty({M, N}, x.options());
+            // Codes, then their scales (rows * K / 2 is a multiple of 2048).
+            const at::Tensor codes = at::empty({rows * (K / 2) + M * (K / 64)}, signs.options());
+            int8_t* packed = static_cast<int8_t*>(codes.data_ptr());
+            const auto fn = rowtiled ? abi.linear_rowtiled : tiled ? abi.linear_tiled : abi.linear;
+            rc = fn(x.data_ptr(), static_cast<const int8_t*>(signs.data_ptr()),
+                    static_cast<const int8_t*>(w.data_ptr()), sw.data_ptr(), out.data_ptr(), packed,
+                    packed + rows * (K / 2), M, N, K, stream_of(dev));
+        }
         if (rc != NV4_OK) Py_RETURN_NONE;
         return THPVariable_Wrap(std::move(out));
     } catch (...) {
@@ -102,8 +113,8 @@ PyObject* dequant_matmul_w4a16(PyObject*, PyObject* const* args, Py_ssize_t n) {
         Py_RETURN_NONE;
     }
     try {
-        const at::Tensor &x = THPVariable_Unpack(args[0]), &qw = THPVariable_Unpack(args[1]),
-                         &qz = THPVariable_Unpack(args[2]), &sc = THPVariable_Unpack(args[3]);
+        const at::Tensor x = THPVariable_Unpack(args[0]), qw = THPVariable_Unpack(args[1]),
+                         qz = THPVariable_Unpack(args[2]), sc = THPVariable_Unpack(args[3]);
         if (!x.is_cuda()) Py_RETURN_NONE;
         const at::Device dev = x.device();
         const at::ScalarType type = x.scalar_type();
@@ -114,25 +125,33 @@ PyObject* dequant_matmul_w4a16(PyObject*, PyObject* const* args, Py_ssize_t n) {
         if (M < 1 || M > mid_max || K < 128 || K % 128 || N < 8 || N % 8 || qw.size(0) * 8 != K || qz.size(0) != G ||
             qz.size(1) != N / 8 || sc.size(0) != G || sc.size(1) != N)
             Py_RETURN_NONE;
-        const c10::DeviceGuard guard(dev);
-        const int code = type == at::kHalf ? NV4_FP16 : NV4_BF16;
-        at::Tensor out = at::empty({M, N}, x.options());
-        const auto* qwp = static_cast<const int32_t*>(qw.data_ptr());
-        const auto* qzp = static_cast<const int32_t*>(qz.data_ptr());
-        void* st = stream_of(dev);
+        at::Tensor out;
         int rc;
-        if (abi.w4a16_one(M, N, K)) {
-            rc = abi.w4a16(x.data_ptr(), code, qwp, qzp, sc.data_ptr(), out.data_ptr(), code, M, N, K, 128, st);
-        } else if (M <= split_max) {
-            const at::Tensor ws = at::empty({(K + slice - 1) / slice * M * N}, x.options().dtype(at::kFloat));
-            rc = abi.w4a16_ws(x.data_ptr(), code, qwp, qzp, sc.data_ptr(), out.data_ptr(), code,
-                              static_cast<float*>(ws.data_ptr()), ws.numel() * 4, M, N, K, 128, st);
-        } else {
-            const int64_t bytes = abi.w4a16_mid_form(M, N, code) ? abi.w4a16_mid_bytes(M, N, K) : -1;
-            if (bytes <= 0) Py_RETURN_NONE;
-            const at::Tensor ws = at::empty({bytes}, x.options().dtype(at::kByte));
-            rc = abi.w4a16_mid(x.data_ptr(), code, qwp, qzp, sc.data_ptr(), out.data_ptr(), code, ws.data_ptr(), bytes,
-                               M, N, K, 128, st);
+        {
+            const NoGil released;
+            const c10::DeviceGuard guard(dev);
+            const int code = type == at::kHalf ? NV4_FP16 : NV4_BF16;
+            const auto* qwp = static_cast<const int32_t*>(qw.data_ptr());
+            const auto* qzp = static_cast<const int32_t*>(qz.data_ptr());
+            void* st = stream_of(dev);
+            if (abi.w4a16_one(M, N, K)) {
+                out = at::empty({M, N}, x.options());
+                rc = abi.w4a16(x.data_ptr(), code, qwp, qzp, sc.data_ptr(), out.data_ptr(), code, M, N, K, 128, st);
+            } else if (M <= split_max) {
+                out = at::empty({M, N}, x.options());
+                const at::Tensor ws = at::empty({(K + slice - 1) / slice * M * N}, x.options().dtype(at::kFloat));
+                rc = abi.w4a16_ws(x.data_ptr(), code, qwp, qzp, sc.data_ptr(), out.data_ptr(), code,
+                                  static_cast<float*>(ws.data_ptr()), ws.numel() * 4, M, N, K, 128, st);
+            } else {
+                const int64_t bytes = abi.w4a16_mid_form(M, N, code) ? abi.w4a16_mid_bytes(M, N, K) : -1;
+                rc = NV4_E_SHAPE;
+                if (bytes > 0) {
+                    out = at::empty({M, N}, x.options());
+                    const at::Tensor ws = at::empty({bytes}, x.options().dtype(at::kByte));
+                    rc = abi.w4a16_mid(x.data_ptr(), code, qwp, qzp, sc.data_ptr(), out.data_ptr(), code,
+                                       ws.data_ptr(), bytes, M, N, K, 128, st);
+                }
+            }
         }
         if (rc != NV4_OK) Py_RETURN_NONE;
         return THPVariable_Wrap(std::move(out));
