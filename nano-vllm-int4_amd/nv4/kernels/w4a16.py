@@ -87,7 +87,7 @@ def mid_form(M, N=None, dtype=torch.float16):
 
 def dequant_matmul_w4a16(x, qweight, qzeros, scales, group_size=128, out=None):
     """x [M,K] bf16/fp16 -> out [M,N] in x's dtype."""
-    if out is None and group_size == 128 and x.is_cuda:
+    if out is None and group_size == 128 and getattr(x, "is_cuda", False):
         # The plain call, natively; None when it is not one (or has more rows).
         native = _lib.ops().dequant_matmul_w4a16(x, qweight, qzeros, scales, SPLIT_MAX_M, SLICE_K, MID_MAX_M)
         if native is not None:

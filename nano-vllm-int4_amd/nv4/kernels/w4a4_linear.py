@@ -33,7 +33,7 @@ def w4a4_linear(x, signs, w_packed, w_scale, *, out=None, out_packed=None, out_s
     row-tiled order ([ceil(M/16)*16, K/2]; tiled weights, M <= 32); None
     chooses it exactly when ``out_packed`` is not given."""
     if out is None and out_packed is None and out_scale is None and weights_f6 is None and packed_rowtiled is None \
-            and x.is_cuda:
+            and getattr(x, "is_cuda", False):
         # The plain call below the fp6 sizes, natively; None when it is not one.
         native = _lib.ops().w4a4_linear(x, signs, w_packed, w_scale, weights_tiled, ROWTILED_MAX_M, PREFILL_MIN_M)
         if native is not None:
