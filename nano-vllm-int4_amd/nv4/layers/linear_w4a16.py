@@ -66,9 +66,12 @@ def fuse_w4a16(linears) -> W4A16Linear:
     column's packing (qzeros packs 8 output channels per int32, so each part's
     N must be a multiple of 8).  The parts' parameters become views into the
     fused tensors, so nothing is stored twice and their state-dict entries
-    keep the reference names and values.  The fused forward equals the
-    concatenation of the parts' forwards bit for bit (columns are computed
-    independently)."""
+    keep the reference names and values.  Columns are computed independently:
+    up to 16 rows and from 33 to 64 the fused forward equals the concatenation
+    of the parts' forwards bit for bit, and at 17 to 32 rows where both take the
+    same kernel (``one_launch``; q/k/v and gate/up of an 8B model do).  Beyond,
+    how K is split (or the library's product) depends on N, and the two may
+    differ by the fp32 sums' order."""
     K = linears[0].in_features
     if any(l.in_features != K or l.group_size != 128 or l.out_features % 8 for l in linears):
         raise ValueError("Fused GPTQ linears need the same input width, group 128 and N % 8 == 0")
