@@ -91,18 +91,13 @@ __device__ __forceinline__ v4i unpack8_x16(uint32_t d0, uint32_t d1) {
 // The compiler would order every later LDS read behind such a load (it tracks
 // few of them apart); with a ring of stages the ones in flight are never the
 // one being read, so the kernel itself waits (lds_ring_barrier) before a stage
-// is read.  Lane l's bytes land at lds + 16 l (4 l); a load past the resource
+// is read.  Lane l's bytes land at lds + 16 l; a load past the resource
 // writes zeros.  A kernel that uses them drains vmcnt before it ends.
 constexpr uint32_t kOutOfRange = 0x7fffff00u;  // scalar offset past every resource
 constexpr uint32_t kRsrcWord3 = 0x00020000u;   // buffer resource word 3 (CDNA): 32-bit data format
 
 __device__ __forceinline__ void lds_load16(const v4u& rsrc, uint32_t voff, uint32_t soff, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff),
-                 "s"(rsrc), "s"(soff)
-                 : "memory");
-}
-__device__ __forceinline__ void lds_load4(const v4u& rsrc, uint32_t voff, uint32_t soff, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(lds), "v"(voff),
                  "s"(rsrc), "s"(soff)
                  : "memory");
 }

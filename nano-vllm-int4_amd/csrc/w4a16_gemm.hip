@@ -22,97 +22,28 @@
 namespace nv4 {
 namespace {
 
-typedef float v2f __attribute__((ext_vector_type(2)));
-typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
-
 template <bool FP16>
 struct W16Traits;
-// The eight nibbles of a qweight word as bytes in k order: p0 = q0..q3,
-// p1 = q4..q7 (two byte permutes of the low and high nibbles).
-__device__ __forceinline__ void nibble_bytes(uint32_t w, uint32_t& p0, uint32_t& p1) {
-    const uint32_t lo = w & 0x0F0F0F0Fu, hi = (w >> 4) & 0x0F0F0F0Fu;  // q0 q2 q4 q6 / q1 q3 q5 q7
-    p0 = __builtin_amdgcn_perm(hi, lo, 0x05010400u);
-    p1 = __builtin_amdgcn_perm(hi, lo, 0x07030602u);
-}
-
 template <>
 struct W16Traits<false> {
     typedef v8bf vec;
     typedef __bf16 elem;
-    struct deq {
-        float s, nzs;  // bf16-rounded scale, -(z+1) * s (exact in fp32)
-    };
     __device__ static inline uint16_t cvt(float f) { return (uint16_t)f32_to_bf16_rne(f); }
     __device__ static inline float scale_of(uint16_t s_f16) {
         // fp16 -> fp32 (exact) -> bf16 (rne), as the reference copies fp16
         // scales into a bf16 buffer.
         return bf16_to_f32(f32_to_bf16_rne((float)__builtin_bit_cast(_Float16, s_f16)));
     }
-    __device__ static inline deq prep(uint16_t s_f16, int zp1) {
-        const float s = scale_of(s_f16);
-        return {s, -((float)zp1 * s)};
-    }
-    // bf16 of (q - z - 1) * s for the word's 8 nibbles: fma(q, s, -(z+1) s)
-    // is exact (every term is a small integer times a bf16), then one
-    // rounding per value, two values per v_cvt_pk_bf16_f32.
-    __device__ static inline vec dequant8(uint32_t w, const deq& d) {
-        uint32_t p0, p1;
-        nibble_bytes(w, p0, p1);
-        float v[8];
-        v[0] = __builtin_fmaf((float)(p0 & 0xffu), d.s, d.nzs);
-        v[1] = __builtin_fmaf((float)((p0 >> 8) & 0xffu), d.s, d.nzs);
-        v[2] = __builtin_fmaf((float)((p0 >> 16) & 0xffu), d.s, d.nzs);
-        v[3] = __builtin_fmaf((float)(p0 >> 24), d.s, d.nzs);
-        v[4] = __builtin_fmaf((float)(p1 & 0xffu), d.s, d.nzs);
-        v[5] = __builtin_fmaf((float)((p1 >> 8) & 0xffu), d.s, d.nzs);
-        v[6] = __builtin_fmaf((float)((p1 >> 16) & 0xffu), d.s, d.nzs);
-        v[7] = __builtin_fmaf((float)(p1 >> 24), d.s, d.nzs);
-        vec r;
-#pragma unroll
-        for (int e = 0; e < 8; e += 2) {
-            const v2bf b = __builtin_convertvector((v2f){v[e], v[e + 1]}, v2bf);
-            r[e] = b[0];
-            r[e + 1] = b[1];
-        }
-        return r;
-    }
 };
 template <>
 struct W16Traits<true> {
     typedef v8h vec;
     typedef _Float16 elem;
-    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-    struct deq {
-        h2 s, nmz;  // (s, s) and (-(1024 + z + 1), ...) in fp16
-    };
     __device__ static inline uint16_t cvt(float f) {
         return __builtin_bit_cast(uint16_t, (_Float16)f);
     }
     __device__ static inline float scale_of(uint16_t s_f16) {
         return (float)__builtin_bit_cast(_Float16, s_f16);
-    }
-    __device__ static inline deq prep(uint16_t s_f16, int zp1) {
-        const _Float16 s = __builtin_bit_cast(_Float16, s_f16);
-        const _Float16 m = (_Float16)(-(1024 + zp1));  // exact: an integer below 2048
-        return {h2{s, s}, h2{m, m}};
-    }
-    // fp16 of (q - z - 1) * s for the word's 8 nibbles: each half is built
-    // as the fp16 1024 + q (bit pattern 0x6400 | q), (1024 + q) - (1024 + z
-    // + 1) is exact, and one packed multiply rounds (q - z - 1) * s once.
-    __device__ static inline vec dequant8(uint32_t w, const deq& d) {
-        uint32_t p0, p1;
-        nibble_bytes(w, p0, p1);
-        const uint32_t m = 0x64646464u;
-        const uint32_t h[4] = {__builtin_amdgcn_perm(m, p0, 0x04010400u), __builtin_amdgcn_perm(m, p0, 0x04030402u),
-                               __builtin_amdgcn_perm(m, p1, 0x04010400u), __builtin_amdgcn_perm(m, p1, 0x04030402u)};
-        vec r;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const h2 v = (__builtin_bit_cast(h2, h[e]) + d.nmz) * d.s;
-            r[2 * e] = v[0];
-            r[2 * e + 1] = v[1];
-        }
-        return r;
     }
 };
 

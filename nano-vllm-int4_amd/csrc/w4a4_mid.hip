@@ -234,6 +234,7 @@ k2_mid(const int8_t* __restrict__ a, const int8_t* __restrict__ w, const uint16_
     constexpr int ROWS = 16 * RB, COLS = 64 * CB;
     constexpr int BUF = MD_SG * RB * 2048;  // widened bytes of a stage
     constexpr int LAG = 2;                  // blocks between a block's MFMAs and its epilogue
+    static_assert(MD_WIN % D == 0, "a window's groups go round the weight ring");
     __shared__ __align__(16) uint8_t st[2][BUF];
     __shared__ int bad_l[4];
 
@@ -346,10 +347,7 @@ k2_mid(const int8_t* __restrict__ a, const int8_t* __restrict__ w, const uint16_
                         __builtin_fmaf((float)acc[x][e], prod[x][e], total[b / CB][b % CB][e]);
             };
             read_a(st[0], std::integral_constant<int, 0>{}, av[0]);
-            constexpr int W = D > MD_WIN ? D / MD_WIN : 1;  // windows per trip
-            for (int gt = 0; gt < G; gt += W * MD_WIN) static_for<0, W>([&](auto wi) {
-                const int g0 = gt + wi * MD_WIN;
-                if (wi > 0 && g0 >= G) return;
+            auto window = [&](int g0) {  // as a lambda: inline in the loop it spills three registers at OCC = 3
                 v4u sa_c[RB], sw_c[CB];
 #pragma unroll
                 for (int i = 0; i < RB; ++i) sa_c[i] = sa_n[i];
@@ -378,10 +376,10 @@ k2_mid(const int8_t* __restrict__ a, const int8_t* __restrict__ w, const uint16_
                     v4i w0[CB], w1[CB];
 #pragma unroll
                     for (int j = 0; j < CB; ++j) {
-                        w0[j] = unpack8_x16(wr[(wi * MD_WIN + u) % D][j][0], wr[(wi * MD_WIN + u) % D][j][1]);
-                        w1[j] = unpack8_x16(wr[(wi * MD_WIN + u) % D][j][2], wr[(wi * MD_WIN + u) % D][j][3]);
+                        w0[j] = unpack8_x16(wr[u % D][j][0], wr[u % D][j][1]);
+                        w1[j] = unpack8_x16(wr[u % D][j][2], wr[u % D][j][3]);
                     }
-                    load_w(g0 + u + D, wr[(wi * MD_WIN + u) % D]);
+                    load_w(g0 + u + D, wr[u % D]);
                     static_for<0, RB * CB>([&](auto B) {
                         constexpr int i = B / CB, j = B % CB, x = u * RB * CB + B;
                         // Of the four scales in the activation side's pair of
@@ -401,7 +399,8 @@ k2_mid(const int8_t* __restrict__ a, const int8_t* __restrict__ w, const uint16_
                     });
                     __builtin_amdgcn_sched_barrier(0);
                 });
-            });
+            };
+            for (int g0 = 0; g0 < G; g0 += MD_WIN) window(g0);
             static_for<MD_WIN * RB * CB - LAG, MD_WIN * RB * CB>(epi);
         }
     }
