@@ -5,9 +5,8 @@
 //   o[i] = softmax_j<=i(scale * q[i] . k[j]) v[j]
 // with GQA (query head h reads KV head h / G), head_dim 128, bf16 in and out.
 //
-// Layout: one workgroup of NW = 8 or 4 waves (launch_fa) per (sequence, KV
-// head, block of QW = 32 NW/G query rows; half of them where two parts of the
-// waves split the keys); wave w takes query head w % G of the group and the 32 query
+// Layout: one workgroup of NW = 8 or 4 waves (launch_fa) per (sequence, KV head,
+// block of QW = 32 NW/G query rows); wave w takes query head w % G of the group and the 32 query
 // rows 32 (w / G) .. of the block, so the G heads of a KV head share every
 // staged key and value.  Keys run in blocks of KB (128 in the 8-wave form,
 // 64 in the 4-wave form) up to the block's last query row; each block is
@@ -53,17 +52,15 @@ static_assert(2 * fa_stage(64) * 2 == 69632 && 2 * fa_stage(128) * 2 == 137216, 
 typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
 typedef float v2f __attribute__((ext_vector_type(2)));
 
-// SPLIT: groups of waves that take equal parts of each key block.
-template <int G, int NW, int FA_KB, int SPLIT = 1>
+template <int G, int NW, int FA_KB>
 __global__ void __launch_bounds__(NW * 64, FA_KB == 64 ? 8 / NW : 1)
 fa_prefill(const uint16_t* __restrict__ q, int64_t q_row, const uint16_t* __restrict__ k, int64_t k_row,
            const uint16_t* __restrict__ v, int64_t v_row, uint16_t* __restrict__ out, int64_t o_row,
            const int32_t* __restrict__ cu, int Hkv, int nqb, float qscale) {
     constexpr int T = NW * 64;
     constexpr int FA_VS = fa_vs(FA_KB), FA_STAGE = fa_stage(FA_KB);
-    constexpr int WK = FA_KB / SPLIT;       // keys of a block per wave
-    constexpr int NC = WK / 32;             // 32-key tiles of them
-    constexpr int QT = NW / (G * SPLIT);    // 32-row query tiles per workgroup
+    constexpr int NC = FA_KB / 32;    // 32-key tiles per block
+    constexpr int QT = NW / G;        // 32-row query tiles per workgroup
     constexpr int QW = 32 * QT;       // query rows per workgroup
     constexpr int KU = FA_KB * FA_D / 8 / T, VU = FA_KB / 2 * FA_D / 8 / T;  // staging units per thread
     static_assert(QT >= 1 && KU * T * 8 == FA_KB * FA_D && VU * T * 16 == FA_KB * FA_D, "staging split");
@@ -78,12 +75,11 @@ fa_prefill(const uint16_t* __restrict__ q, int64_t q_row, const uint16_t* __rest
 
     const int t = threadIdx.x, lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int hq = kvh * G + wave % G, qt = wave / G % QT, part = wave / (G * QT);
+    const int hq = kvh * G + wave % G, qt = wave / G;
     const int rc = lane & 31, hh = lane >> 5;
     const int qr = q0 + 32 * qt + rc;    // this lane's query row (rows >= L are computed, not stored)
     const int lim = min(qr, L - 1);      // last key this row attends to
     const int wave_q0 = q0 + 32 * qt;    // the wave's first query row
-    const int wave_key = part * WK;      // the wave's first key of a block
 
     // Q^T operands, 16-dim step s: dims 16 s + 8 hh .. +7 of the lane's row.
     v4u qv[8];
@@ -141,8 +137,8 @@ fa_prefill(const uint16_t* __restrict__ q, int64_t q_row, const uint16_t* __rest
     for (int dt = 0; dt < 4; ++dt) o[dt] = v16f{};
 
     auto compute = [&](int kb) {
-        const uint16_t* Ks = lds + (kb & 1) * FA_STAGE + wave_key * FA_KS;
-        const uint16_t* Vt = lds + (kb & 1) * FA_STAGE + FA_KB * FA_KS + wave_key;
+        const uint16_t* Ks = lds + (kb & 1) * FA_STAGE;
+        const uint16_t* Vt = Ks + FA_KB * FA_KS;
         v16f sc[NC];
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
@@ -157,8 +153,8 @@ fa_prefill(const uint16_t* __restrict__ q, int64_t q_row, const uint16_t* __rest
         }
         // Causal and sequence-end mask, only in blocks that reach past the
         // wave's first query row or the sequence (uniform over the wave).
-        const int key0 = kb * FA_KB + wave_key;
-        if (key0 + WK - 1 > wave_q0 || key0 + WK > L) {
+        const int key0 = kb * FA_KB;
+        if (key0 + FA_KB - 1 > wave_q0 || key0 + FA_KB > L) {
 #pragma unroll
             for (int c = 0; c < NC; ++c)
 #pragma unroll
@@ -173,8 +169,8 @@ fa_prefill(const uint16_t* __restrict__ q, int64_t q_row, const uint16_t* __rest
 #pragma unroll
             for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sc[c][i]);
         mx = fmaxf(mx, __shfl_xor(mx, 32));
-        const float mn = fmaxf(m, mx);  // with key 0 (never masked) finite from the first block on
-        const float off = SPLIT > 1 && mn == -__builtin_inff() ? 0.0f : -mn * qscale;
+        const float mn = fmaxf(m, mx);  // finite from the first block on (key 0 is never masked)
+        const float off = -mn * qscale;
         const float corr = __builtin_amdgcn_exp2f(__builtin_fmaf(m, qscale, off));
         m = mn;
         // P^T operands: step t of tile c takes values 8t .. 8t + 7.
@@ -223,42 +219,12 @@ fa_prefill(const uint16_t* __restrict__ q, int64_t q_row, const uint16_t* __rest
         // The next block's loads fly during this block's arithmetic; past the
         // last block they reload it into the unused stage.
         load(min(kb + 1, nkb - 1));
-        // A part past the wave's last row is all masked (uniform over the wave).
-        if (SPLIT == 1 || kb * FA_KB + wave_key <= wave_q0 + 31) compute(kb);
+        compute(kb);
         store((kb + 1) & 1);
         __syncthreads();
     }
 
     l += __shfl_xor(l, 32);
-    if constexpr (SPLIT > 1) {  // the second part's max, sum and output join the first's
-        static_assert(SPLIT == 2, "two parts");
-        constexpr int HALF = T / 2;
-        static_assert(18 * HALF * 16 <= 2 * FA_STAGE * 2, "the exchange fits the stages");
-        v4f* xo = reinterpret_cast<v4f*>(lds);
-        float* xm = reinterpret_cast<float*>(lds) + 16 * HALF * 4;
-        const int slot = t % HALF;
-        if (part) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i)
-                xo[i * HALF + slot] = v4f{o[i >> 2][4 * (i & 3)], o[i >> 2][4 * (i & 3) + 1],
-                                          o[i >> 2][4 * (i & 3) + 2], o[i >> 2][4 * (i & 3) + 3]};
-            xm[slot] = m;
-            xm[HALF + slot] = l;
-        }
-        __syncthreads();
-        if (part) return;
-        const float m1 = xm[slot], mn = fmaxf(m, m1), off = -mn * qscale;
-        const float c0 = __builtin_amdgcn_exp2f(__builtin_fmaf(m, qscale, off));
-        const float c1 = __builtin_amdgcn_exp2f(__builtin_fmaf(m1, qscale, off));
-        l = __builtin_fmaf(l, c0, xm[HALF + slot] * c1);
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const v4f p = xo[i * HALF + slot];
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                o[i >> 2][4 * (i & 3) + e] = __builtin_fmaf(o[i >> 2][4 * (i & 3) + e], c0, p[e] * c1);
-        }
-    }
     const float inv = 1.0f / l;
     if (qr < L) {
         uint16_t* op = out + (int64_t)(start + qr) * o_row + (int64_t)hq * FA_D + 4 * hh;
@@ -274,20 +240,15 @@ fa_prefill(const uint16_t* __restrict__ q, int64_t q_row, const uint16_t* __rest
     }
 }
 
-// Three forms (us, back to back, 32 query heads over 8 KV heads unless said otherwise):
+// Two forms (us on inputs from memory, 32 query heads over 8 KV heads unless said
+// otherwise):
 //  * eight waves, 32 * 8/G query rows: half the staging per row, for grids that
-//    fill the CUs with long prompts (4096 tokens 159 against 181 with four
-//    waves; 2 x 2048 90 against 95), and grids of exactly one workgroup per CU
-//    (16 heads over 8, 4 x 1024: 40 against 43);
+//    fill the CUs with long prompts (4096 tokens 160 against 180 with four
+//    waves; 4 x 2048 177 against 184) and grids of exactly one workgroup per CU;
 //  * four waves, two workgroups per CU: grids that would leave CUs idle, and
 //    prompts of up to 1024 tokens in larger ones, where the fixed cost of a
-//    workgroup and the last wave of them count (32 x 128 tokens 36.0 -> 27.5,
-//    8 x 400 40.2 -> 34.8, 32 x 512 184 -> 151, 8 x 1024 121 -> 111);
-//  * eight waves of which each half takes half of every key block, for the same
-//    rows as four: up to 1.5 workgroups per CU the longest extent bounds the
-//    time (1500 tokens 43.1 -> 37.5, cold 42.1 -> 40.4, 1100 33.8 -> 30.6; 16 heads over 8, 3000
-//    tokens 76 -> 63; with 2 per CU, 2000 tokens, equal; 4 x 1024 of 16 heads over
-//    8 42.5 -> 52.7), and not up to 1024 tokens (512: 17.1 against 17.5).
+//    workgroup and the last wave of them count (32 x 128 tokens 37.5 -> 30.6, 8
+//    x 400 45.1 -> 36.9, 32 x 512 184 -> 146, 8 x 1024 123 -> 113).
 constexpr int64_t FA_SHORT = 1024;
 template <int G>
 hipError_t launch_fa(const uint16_t* q, int64_t q_row, const uint16_t* k, int64_t k_row, const uint16_t* v,
@@ -302,13 +263,6 @@ hipError_t launch_fa(const uint16_t* q, int64_t q_row, const uint16_t* k, int64_
                            k, k_row, v, v_row, out, o_row, cu, Hkv, nqb, qscale);
     } else {
         const int nqb = (int)((max_seqlen + 32 * (NW / G) - 1) / (32 * (NW / G)));
-        if constexpr (G <= 4) {
-            if (max_seqlen > FA_SHORT && 2 * (int64_t)nqb * Hkv * B <= 3 * cus) {
-                hipLaunchKernelGGL((fa_prefill<G, 8, 128, 2>), dim3((unsigned)(nqb * Hkv), (unsigned)B), dim3(512), 0,
-                                   st, q, q_row, k, k_row, v, v_row, out, o_row, cu, Hkv, nqb, qscale);
-                return hipGetLastError();
-            }
-        }
         hipLaunchKernelGGL((fa_prefill<G, NW, 64>), dim3((unsigned)(nqb * Hkv), (unsigned)B), dim3(NW * 64), 0, st, q,
                            q_row, k, k_row, v, v_row, out, o_row, cu, Hkv, nqb, qscale);
     }

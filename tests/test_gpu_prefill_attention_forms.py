@@ -1,7 +1,7 @@
 """GPU parity of the prefill attention forms (nanovllm/layers/attention.py:64-70)
-where the launch rule changes: prompts past 1024 tokens whose key blocks two
-halves of a workgroup share, ragged batches whose short members end inside a
-first half, and larger grids of short prompts on four waves.
+where the launch rule changes: single prompts past 1024 tokens, ragged batches
+whose short members end inside a first block, and larger grids of short prompts
+on four waves.
 
 Reference: float64 on the CPU.  Tolerance: P rounds to bf16 (2^-8 of each
 weight, hence of the largest |v| of the head) and the result once more (2^-8 of
