@@ -244,11 +244,13 @@ fa_prefill(const uint16_t* __restrict__ q, int64_t q_row, const uint16_t* __rest
 // otherwise):
 //  * eight waves, 32 * 8/G query rows: half the staging per row, for grids that
 //    fill the CUs with long prompts (4096 tokens 160 against 180 with four
-//    waves; 4 x 2048 177 against 184) and grids of exactly one workgroup per CU;
+//    waves; 4 x 2048 177 against 184; 16 heads over 8, 2 x 2048 74 against 77);
 //  * four waves, two workgroups per CU: grids that would leave CUs idle, and
-//    prompts of up to 1024 tokens in larger ones, where the fixed cost of a
-//    workgroup and the last wave of them count (32 x 128 tokens 37.5 -> 30.6, 8
-//    x 400 45.1 -> 36.9, 32 x 512 184 -> 146, 8 x 1024 123 -> 113).
+//    prompts of up to 1024 tokens in any, where the fixed cost of a workgroup and
+//    the last wave of them count (32 x 128 tokens 37.5 -> 30.6, 8 x 400 45.1 ->
+//    36.9, 32 x 512 184 -> 146, 8 x 1024 123 -> 113; with eight-wave grids of one
+//    workgroup per CU 8 x 193 21.0 -> 16.6, 16 x 128 20.9 -> 17.2, 4 x 512 29.4
+//    -> 28.6, 2 x 1024 42.8 -> 43.9, 8 heads over 8 at 8 x 1024 41.2 -> 43.5).
 constexpr int64_t FA_SHORT = 1024;
 template <int G>
 hipError_t launch_fa(const uint16_t* q, int64_t q_row, const uint16_t* k, int64_t k_row, const uint16_t* v,
@@ -256,8 +258,7 @@ hipError_t launch_fa(const uint16_t* q, int64_t q_row, const uint16_t* k, int64_
                      int Hkv, float qscale, hipStream_t st) {
     constexpr int NW = G > 4 ? 8 : 4;
     const int64_t nqb8 = (max_seqlen + 32 * (8 / G) - 1) / (32 * (8 / G));
-    const int64_t cus = device_cu_count(), grid8 = nqb8 * Hkv * B;
-    if (G > 4 || grid8 == cus || (grid8 > cus && max_seqlen > FA_SHORT)) {
+    if (G > 4 || (nqb8 * Hkv * B >= device_cu_count() && max_seqlen > FA_SHORT)) {
         const int nqb = (int)nqb8;
         hipLaunchKernelGGL((fa_prefill<G, 8, 128>), dim3((unsigned)(nqb * Hkv), (unsigned)B), dim3(512), 0, st, q, q_row,
                            k, k_row, v, v_row, out, o_row, cu, Hkv, nqb, qscale);
