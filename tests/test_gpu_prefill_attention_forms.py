@@ -5,7 +5,10 @@ on four waves.
 
 Reference: float64 on the CPU.  Tolerance: P rounds to bf16 (2^-8 of each
 weight, hence of the largest |v| of the head) and the result once more (2^-8 of
-it); an output is a convex combination of v, so 2^-7 of the head's largest |v|."""
+it); an output is a convex combination of v, so 2^-7 of the head's largest |v|.
+Over many keys of independent v both roundings and the result are random sums of
+the same weights, so by the 2-norm over a head's rows the error stays below 2^-7
+of the result, in the first 512 rows and in the later ones, whose outputs are the smallest."""
 import pytest
 import torch
 
@@ -16,7 +19,8 @@ DEV = "cuda:0"
 
 
 @pytest.mark.parametrize("hq,hkv,lens", [(32, 8, [1025]), (32, 8, [1499]), (16, 8, [1100, 3, 65]), (8, 8, [1300]),
-                                         (4, 1, [1200, 1, 31, 129]), (8, 2, [300] * 60), (32, 8, [130] * 16)])
+                                         (4, 1, [1200, 1, 31, 129]), (8, 2, [300] * 60), (32, 8, [130] * 16),
+                                         (32, 8, [200] * 8)])
 def test_against_64_bits(hq, hkv, lens):
     print(f"[prefill_forms] hq={hq} hkv={hkv} lens={lens[:4]} x{len(lens)}", flush=True)
     g = torch.Generator("cpu").manual_seed(len(lens) + lens[0])
@@ -33,4 +37,7 @@ def test_against_64_bits(hq, hkv, lens):
             scores = q[a:b, h].double() @ kh.T * 128**-0.5
             scores.masked_fill_(torch.ones(b - a, b - a, dtype=torch.bool).triu(1), float("-inf"))
             ref = scores.softmax(-1) @ vh
-            assert (out[a:b, h].double() - ref).abs().max() <= 2.0**-7 * vh.abs().max()
+            error = out[a:b, h].double() - ref
+            assert error.abs().max() <= 2.0**-7 * vh.abs().max()
+            for rows in (slice(0, 512), slice(512, None)):
+                assert error[rows].norm() <= 2.0**-7 * ref[rows].norm()
