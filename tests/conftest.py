@@ -28,7 +28,7 @@ def _ensure_built():
     if not (ROOT / "oracle" / "liboracle.so").exists():
         subprocess.run(["make", "-C", str(ROOT / "oracle")], check=True, stdout=subprocess.DEVNULL)
     if not (PKG / "nv4" / "libnv4.so").exists() or not (PKG / "nv4" / "_ops.so").exists():
-        subprocess.run(["make", "-C", str(PKG), "-j8"], check=True, stdout=subprocess.DEVNULL)
+        subprocess.run(["make", "-C", str(PKG), "-j8", f"PYTHON={sys.executable}"], check=True, stdout=subprocess.DEVNULL)
 
 
 _ensure_built()
