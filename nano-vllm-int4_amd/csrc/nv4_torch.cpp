@@ -143,7 +143,12 @@ PyObject* dequant_matmul_w4a16(PyObject*, PyObject* const* args, Py_ssize_t n) {
                 rc = abi.w4a16_ws(x.data_ptr(), code, qwp, qzp, sc.data_ptr(), out.data_ptr(), code,
                                   static_cast<float*>(ws.data_ptr()), ws.numel() * 4, M, N, K, 128, st);
             } else {
-                const int64_t bytes = abi.w4a16_mid_form(M, N, code) ? abi.w4a16_mid_bytes(M, N, K) : -1;
+                // (weights off the alignment that every form past 64 rows asks of
+                // them are the general path's to refuse)
+                const bool aligned = !(reinterpret_cast<uintptr_t>(qwp) % 16 ||
+                                       reinterpret_cast<uintptr_t>(sc.data_ptr()) % 16);
+                const int64_t bytes =
+                    aligned && abi.w4a16_mid_form(M, N, code) ? abi.w4a16_mid_bytes(M, N, K) : -1;
                 rc = NV4_E_SHAPE;
                 if (bytes > 0) {
                     out = at::empty({M, N}, x.options());

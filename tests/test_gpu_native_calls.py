@@ -59,6 +59,24 @@ def test_w4a16_same_bits(M, K, dtype):
     assert got is not None and torch.equal(got, want)
 
 
+@pytest.mark.parametrize("which,words,taken", [(1, 2, False), (1, 1, False), (3, 2, False), (3, 4, False),
+                                               (0, 4, True)])
+def test_w4a16_off_alignment(which, words, taken):
+    """Tensors that begin inside a 16-byte unit, past 64 rows: rows are taken,
+    weights refused, whichever path the call goes."""
+    args = list(w4a16_args(100, 136, 1024, torch.bfloat16))
+    t = args[which]
+    buf = torch.empty(t.numel() + words, dtype=t.dtype, device=DEV)
+    args[which] = buf[words:].view(t.shape).copy_(t)
+    out = torch.empty(100, 136, dtype=torch.bfloat16, device=DEV)
+    if taken:
+        assert torch.equal(dequant_matmul_w4a16(*args), dequant_matmul_w4a16(*args, out=out))
+    else:
+        for more in ({}, {"out": out}):
+            with pytest.raises(ValueError, match="misaligned"):
+                dequant_matmul_w4a16(*args, **more)
+
+
 def test_other_calls_stay_with_the_general_path():
     class Sub(torch.Tensor):
         pass
