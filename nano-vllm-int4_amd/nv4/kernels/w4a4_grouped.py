@@ -49,24 +49,37 @@ PATHS = ("int8", "fp8", "fp6")
 
 
 # No size below this M runs on the fp6 matrix cores (``use_prefill_path``).
-PREFILL_MIN_M = 448
+PREFILL_MIN_M = 449
 
 
-def use_prefill_path(M, N, K):
+def use_prefill_path(M, N, K, kept=False):
     """Prefill-sized GEMMs run on the fp6 matrix cores (``nv4_w4a4_gemm_f6``).
     The operand conversion costs about 1.25 (M + N) K bytes of traffic and one
-    launch.  Against the int8 kernels it pays from M = 448 on gate_up (us per
-    call at 383 / 448 / 512: 65, 77, 81 int8 against 72, 74, 78), from M = 768
-    on the narrower projections above 4096 x 4096 (qkv at 700 / 777: 36, 43
-    against 42, 42; down at 700 / 832: 65, 71 against 67, 69) and past M = 1024
-    on all others (o at 777 / 1024: 30.5, 31.7 against 32.4, 31.7)."""
-    nk = N * K
-    return M > 1024 or (M >= 768 and nk > 4096 * 4096) or (M >= PREFILL_MIN_M and nk >= 4096 * 24576)
+    launch, of which weights kept in that form (``kept``) leave 1.25 M K.  us per
+    call, int8 / fp6, on weights from memory:
+
+    * past M = 1024 everywhere (4096 x 4096 at 1024: 28.3 / 31.1, at 1280: 41.6 /
+      39.1, at 2048: 54.1 / 44.0);
+    * past 768 rows above 4096 x 4096 (6144 x 4096 at 768: 34.2 / 41.2, at 832:
+      42.3 / 41.2; 4096 x 12288: 62.1 / 66.6 and 69.0 / 67.4; 12288 x 4096: 63.0 /
+      63.4; 16384 x 4096: 77.5 / 71.7);
+    * past 512 rows from 4096 x 20480 (20480 x 4096 at 512: 67.2 / 71.9, at 640:
+      92.2 / 83.1; 8192 x 12288: 76.6 / 82.2 and 115 / 103; 24576 x 4096 at 576: 97.8
+      / 85.5);
+    * past 448 rows where the 128 x 128 tiles are three per CU or more (24576 x 4096
+      at 448: 73.0 / 73.3, at 512: 77.9 / 74.5; 32768 x 4096 at 512: 105 / 97.8;
+      two and a half and fewer: the sizes above);
+    * with kept weights past 512 rows above 4096 x 4096 (6144 x 4096 at 576: 26.8
+      / 25.3; 4096 x 12288 at 512: 45.5 / 57.3, at 576: 60.8 / 57.5)."""
+    nk, tiles = N * K, (M + 127) // 128 * ((N + 127) // 128)
+    return (M > 1024 or (M > 768 and nk > 4096 * 4096)
+            or (M > 512 and (nk >= 4096 * 20480 or (kept and nk > 4096 * 4096)))
+            or (M >= PREFILL_MIN_M and tiles >= 3 * 256))
 
 
-def _resolve_path(path, M, N, K):
+def _resolve_path(path, M, N, K, kept=False):
     if path is None:
-        return "fp6" if use_prefill_path(M, N, K) else "int8"
+        return "fp6" if use_prefill_path(M, N, K, kept) else "int8"
     if path not in PATHS:
         raise ValueError(f"path must be None or one of {PATHS}")
     return path
@@ -127,7 +140,7 @@ def _check_weights_f6(weights_f6, N, K, device):
 def _launch(a_packed, w_packed, a_scale, w_scale, out, output_fp32, weight_grouped, weights_tiled=False, path=None,
             weights_f6=None):
     M, N, K = a_packed.shape[0], w_packed.shape[0], a_packed.shape[1] * 2
-    path = _resolve_path(path, M, N, K)
+    path = _resolve_path(path, M, N, K, weights_f6 is not None)
     lib = _lib.load()
     stream = torch.cuda.current_stream(a_packed.device).cuda_stream
     with torch.cuda.device(a_packed.device):

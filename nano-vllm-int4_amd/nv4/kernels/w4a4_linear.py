@@ -75,7 +75,7 @@ def w4a4_linear(x, signs, w_packed, w_scale, *, out=None, out_packed=None, out_s
     if any(not t.is_cuda or not t.is_contiguous() or t.device != dev for t in tensors):
         raise ValueError("All tensors must be contiguous on one CUDA device")
     _check_weights_f6(weights_f6, N, K, dev)
-    if use_prefill_path(M, N, K):
+    if use_prefill_path(M, N, K, weights_f6 is not None):
         # Prefill-sized M: K1, then the grouped GEMM on the fp6 matrix cores.
         rht_quant_pack(x, signs, out_packed=out_packed, out_scale=out_scale)
         _launch(out_packed, w_packed, out_scale, w_scale, out, False, True, weights_tiled, path="fp6",
