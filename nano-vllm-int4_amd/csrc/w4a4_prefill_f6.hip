@@ -37,13 +37,14 @@
 // go through a three-stage LDS ring, loaded three groups ahead, with one
 // barrier per group; a wave reads an operand of the next group right after
 // its last use in this one, and every MFMA is followed by a third of the
-// previous block's fma chain, so LDS, matrix cores and vector ALUs work at the
-// same time.  Against a two-stage ring with a group's reads, MFMAs and fmas in
-// turn (us per call with the conversion): M = 4096 qkv 113 -> 103, o 78.8 ->
-// 72.9, gate_up 402 -> 390, down 206 -> 196; M = 1024 o 34.3 -> 30.4, down 82 ->
-// 69.  What bounds it now: the chip's power at large M (gate_up at 4096 rows
-// takes 330 us on zero codes and 286 without the operand loads), one
-// workgroup's own 0.42 us per group while tiles are fewer than CUs.
+// previous block's fma chain.  Against a two-stage ring with a group's reads,
+// MFMAs and fmas in turn (us per call with the conversion): M = 4096 qkv 113 ->
+// 103, o 78.8 -> 72.9, gate_up 402 -> 390, down 206 -> 196; M = 1024 o 34.3 ->
+// 30.4, down 82 -> 69.  What bounds it now: matrix cores and vector ALUs in
+// turn (42 and 43 % of the cycles of gate_up at 4096 rows, LDS 66 %) at the
+// clock that the chip's power leaves, 1.95 GHz (330 us on zero codes, 286
+// without the operand loads); one workgroup's own 0.42 us per group while
+// tiles are fewer than CUs.
 #include "nv4_common.h"
 
 namespace nv4 {
