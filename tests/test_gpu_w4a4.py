@@ -340,9 +340,10 @@ def extreme_scales(rng, rows, G, frac=0.05):
 @pytest.mark.parametrize("M,N,K,rows_special", [(200, 264, 1024, True), (257, 392, 2048, False),
                                                  (150, 136, 12288, True), (130, 400, 1024, False)])
 def test_k2_prefill_extreme_scales(M, N, K, rows_special):
-    """Prefill tiles whose scales leave the range where the kernel folds the
-    x256 of the widened nibbles into the activation scale must take the
-    literal per-group sequence; tiles next to them keep the short form.
+    """Tiles past the decode sizes (here the mid-sized kernels'; the 128 x 128
+    ones: test_gpu_k2_prefill.py) whose scales leave the range where the kernel
+    folds the x256 of the widened nibbles into a scale must take the literal
+    per-group sequence; tiles next to them keep the short form.
     Only some rows (or some columns) carry the special values, so both forms
     run in one launch.  Bit-exact in bf16 and fp32."""
     print(f"[k2-extreme] M={M} N={N} K={K}", flush=True)
@@ -375,9 +376,9 @@ def test_k2_prefill_extreme_scales(M, N, K, rows_special):
 
 @pytest.mark.parametrize("M,N,K", [(1000, 1032, 512), (300, 520, 1024), (4096, 264, 2048)])
 def test_k2_prefill_tile_orders(M, N, K):
-    """Every output of prefill launches whose tile counts are (72, 15, 96) --
-    divisible by the 8 XCDs or not -- so every tile of both orderings is
-    written exactly once and lands where it belongs."""
+    """Every output of launches on the mid-sized and fp6 tiles, counts divisible
+    by the 8 XCDs or not, so every tile of both orderings is written exactly once
+    and lands where it belongs (the 128 x 128 int8 tiles: test_gpu_k2_prefill.py)."""
     run_case(M, N, K, 7000 + M + N)
 
 
